@@ -56,10 +56,8 @@ __device__ inline void wave_sum_segment(const double* __restrict__ partial, int3
         t1 += b[u];
       }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    t0 += __shfl_down(t0, o, 64);
-    t1 += __shfl_down(t1, o, 64);
-  }
+  t0 = wave_sum(t0);
+  t1 = wave_sum(t1);
 }
 
 // one wavefront per case: sum its partials and run its scalar update
@@ -996,8 +994,19 @@ static void bcg(BSolver<T>& S, int precon, const T* b, T* x0, int itmax, double 
                        Sd, r, zd, (const T*)nullptr, F.start());
     F.done(FIN_CG_INIT);
   }
-  int parity = 0;
   xcal_ctx* c = S.m->ctx;
+  bool resident = false;
+  if (!dilu && !graphs_enabled(c)) {  // the whole solve in one resident launch (persist.h)
+    F.flush();
+    PersistLease lease;
+    resident = persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease);
+    if (resident && !bread(S)) {  // its waits were given up: start over by launches
+      persist_failed(S.m);
+      bcg(S, precon, b, x0, itmax, atol, rtol, frozen, xsol);
+      return;
+    }
+  }
+  int parity = 0;
   auto iteration = [&]() {
     T* pold = parity ? pb : pa;
     T* pnew = parity ? pa : pb;
@@ -1043,8 +1052,9 @@ static void bcg(BSolver<T>& S, int precon, const T* b, T* x0, int itmax, double 
   const auto key = graph_key(S, 0, precon, nullptr);
   // fused chains carry their pending finalize between launches, so they are
   // not captured
-  brun(S, 4, iteration, graphs_enabled(c) && !F.on ? &key : nullptr, &parity,
-       [&] { F.flush(); });
+  if (!resident)
+    brun(S, 4, iteration, graphs_enabled(c) && !F.on ? &key : nullptr, &parity,
+         [&] { F.flush(); });
   if (x0) hipLaunchKernelGGL(kb_add, dim3(grid_for(n)), dim3(kBlock), 0, S.s, n, (const double*)x,
                              (double*)x0);
   if (xsol) *xsol = x;

@@ -1091,6 +1091,7 @@ static xcal_mesh* upload_mesh(xcal_ctx* ctx, HostMesh& M) {
     m->roww = std::max(m->roww, (M.rend[c] - M.rbeg[c]) / kSlice);
   const char* nofuse = std::getenv("XCAL_NO_FUSE");
   m->fuse = !(nofuse && *nofuse == '1');
+  persist_configure(m.get());
   m->nbcell = M.nbcell;
   m->n_patches = M.n_patches;
   m->patch_first = M.patch_first;

@@ -480,9 +480,43 @@ __device__ inline int32_t level_pos(int32_t cnt, int32_t& end) {
   return (int32_t)(c0 + (int64_t)l * blockDim.x + threadIdx.x);
 }
 
-// Deterministic block-level sum (wave shuffles + LDS), result in thread 0.
+// v of the lane `O` above, as lane 0's sum tree needs it (other lanes may get
+// other values): O = 32 and 16 by swapping halves and rows of the wavefront,
+// 8, 4, 2, 1 by a DPP shift inside a row of 16.  A __shfl_down goes through
+// the LDS crossbar, two dependent round trips per double.
+template <int O>
+__device__ inline double lane_above(double v) {
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  unsigned l, h;
+  if constexpr (O == 32) {
+    l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false)[1];
+    h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false)[1];
+  } else if constexpr (O == 16) {
+    l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false)[1];
+    h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false)[1];
+  } else {
+    l = (unsigned)__builtin_amdgcn_update_dpp(0, (int)lo, 0x100 | O, 0xf, 0xf, true);
+    h = (unsigned)__builtin_amdgcn_update_dpp(0, (int)hi, 0x100 | O, 0xf, 0xf, true);
+  }
+  return __hiloint2double((int)h, (int)l);
+}
+
+// Sum over a wavefront, all lanes active; the result is in lane 0 only.  Lane
+// 0's tree adds lane i + o to lane i for o = 32, 16, 8, 4, 2, 1, the order of
+// six __shfl_down steps bit for bit.
+__device__ inline double wave_sum(double v) {
+  v += lane_above<32>(v);
+  v += lane_above<16>(v);
+  v += lane_above<8>(v);
+  v += lane_above<4>(v);
+  v += lane_above<2>(v);
+  v += lane_above<1>(v);
+  return v;
+}
+
+// Deterministic block-level sum (wave sums + LDS), result in thread 0.
 __device__ inline double block_sum(double v, double* lds) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+  v = wave_sum(v);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) lds[wid] = v;
   __syncthreads();

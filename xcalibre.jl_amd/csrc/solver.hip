@@ -999,6 +999,18 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
                        r, zd, (const T*)nullptr, S.partial);
     finalize_launch(S, S.grid, FIN_CG_INIT);
   }
+  KS st{};
+  if (!dilu) {  // small meshes: the whole solve in one resident launch (persist.h)
+    PersistLease lease;
+    if (persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease)) {
+      st = read_state(S);
+      if (st.stop == STOP_NONE) {  // its waits were given up: start over by launches
+        persist_failed(S.m);
+        return cg(S, precon, b, x0, itmax, atol, rtol, niter, xsol);
+      }
+      *S.cg_batch = st.iter;
+    }
+  }
   int parity = 0;
   // The cone sweeps read the old r of other workgroups' rows while the fused
   // update writes the new one, so r alternates between two vectors there.
@@ -1072,7 +1084,7 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
       F.done(pu, S.grid, FIN_CG_ITER);
     }
   };
-  KS st = read_state(S);
+  if (st.stop == STOP_NONE) st = read_state(S);
   if (st.stop == STOP_NONE)
     run_batches(S, S.cg_batch, 4, iteration, st, [&] {
       F.flush();

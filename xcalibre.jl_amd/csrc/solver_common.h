@@ -191,8 +191,7 @@ __device__ inline double block_sum_rows(const double (&v)[RW], double* lds) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int j = 0; j < RW; ++j) {
-    double x = v[j];
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
+    const double x = wave_sum(v[j]);
     if (lane == 0) lds[(j * (int)blockDim.x + (int)threadIdx.x) >> 6] = x;
   }
   __syncthreads();
@@ -414,6 +413,23 @@ __device__ inline void bwd_row(const BwdK<T>& W, int32_t pos, int64_t e0, int32_
   if (DOT == 4) { s0 += dd(zi, zi); s1 += dd(dvi, zi); }
 }
 
+
+// ------------------------------------------------------------ resident CG
+// Workgroups of resident launches in flight (persist.hip): held from the
+// launch until its stream has been waited for.
+struct PersistLease {
+  int dev = 0, n = 0;
+  bool acquire(int device, int nwg, int cap);
+  void release();
+  PersistLease() = default;
+  PersistLease(const PersistLease&) = delete;
+  PersistLease& operator=(const PersistLease&) = delete;
+  ~PersistLease() { release(); }
+};
+template <class T>
+bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T* z, KS* ks,
+                PersistLease& lease);
+void persist_failed(const xcal_mesh* m);
 
 // ----------------------------------------------------- kernel timing hook
 // Timing-only events: without the system-scope fence, recording one does not

@@ -139,6 +139,10 @@ struct DBuf {
 
 }  // namespace xcal
 
+namespace xcal {
+struct PersistPlan;  // persist.hip
+}
+
 // ----------------------------------------------------------------- handles
 struct xcal_ctx {
   int device = 0;
@@ -207,6 +211,11 @@ struct xcal_mesh {
   int64_t nzlen = 0;  // storage length including slice padding
   int32_t roww = 0;   // most entries in one row
   bool fuse = true;   // fused Krylov finalizes allowed (XCAL_NO_FUSE=1 at creation: off)
+  // Resident CG (persist.h): allowed, ticks (100 MHz) a wait may take, and
+  // its plan (made at the first solve)
+  mutable bool persist_on = true;
+  long long persist_ticks = 100000000;
+  mutable std::shared_ptr<xcal::PersistPlan> persist;
   xcal::DBuf<int32_t> rbeg, rend, colval, trans;
   xcal::DBuf<int32_t> sinfo;  // per slice of kSlice rows: first slot, width (entries)
   // DILU level schedules: forward level l = device rows
@@ -320,6 +329,7 @@ struct xcal_eqn {
   xcal::DBuf<double> ncflux;  // non-orthogonal correction per internal face
   xcal::DBuf<double> fpart;   // fused finalizes: two partial areas
   xcal::DBuf<char> fstate;    // fused finalizes: two more Krylov states
+  xcal::DBuf<unsigned long long> parea;  // resident CG: published sums, abort word
   void* kstate_host = nullptr;  // pinned copy
   int cg_batch = 0, bi_batch = 0;   // iterations of the last solve (first-batch size)
   // mixed precision: FP32 copies of the matrix and preconditioner, workspace
@@ -379,6 +389,7 @@ struct BCsK {
 };
 
 void make_sweep_plans(xcal_mesh* m, int small);
+void persist_configure(xcal_mesh* m);
 // meshes built on the host first (server admission), uploaded later
 struct PreparedMesh;
 // Host build of one mesh or a batch.  With `ingest`, the CSR pattern, slot
