@@ -352,9 +352,14 @@ int xcal_eqn_download(const xcal_eqn* e, int32_t which, int32_t comp, double* nz
     XCAL_CHECK(which == 0 || (which == 1 && e->vector), "which: 0 = A, 1 = A0 (vector only)");
     XCAL_CHECK(comp >= 0 && comp < (e->vector ? 3 : 1), "component out of range");
     const xcal_mesh* m = e->mesh;
-    if (nzval) download_permuted(m, m->nzperm, which ? e->nzval0.p : e->nzval.p, nzval, m->nnz,
-                                  m->nzlen);
-    if (b) download_permuted(m, m->cperm, e->bc(comp), b, m->n);
+    if (nzval) {
+      std::vector<double> t(m->nzlen);
+      XCAL_HIP(hipMemcpyAsync(t.data(), which ? e->nzval0.p : e->nzval.p,
+                              sizeof(double) * m->nzlen, hipMemcpyDeviceToHost, m->ctx->stream));
+      XCAL_HIP(hipStreamSynchronize(m->ctx->stream));
+      for (int64_t k = 0; k < m->nnz; ++k) nzval[k] = t[m->nzperm[k]];
+    }
+    if (b) download_permuted(m, m->cperm_d.p, e->bc(comp), b, m->n);
     return 0;
   });
 }

@@ -648,9 +648,8 @@ void simple_case_field(const xcal_simple* S, int which, int k, double* host) {
                                                      : nullptr;
   XCAL_CHECK(f, "unknown cell field selector (or no turbulence model)");
   const int64_t c0 = m->case_cell[k], nk = m->case_cell[k + 1] - c0;
-  const std::vector<int32_t> perm(m->cperm.begin() + c0, m->cperm.begin() + c0 + nk);
   for (int c = 0; c < f->ncomp; ++c)
-    download_permuted(m, perm, f->comp(c), host + (int64_t)c * nk, nk, f->len);
+    download_permuted(m, m->cperm_d.p + c0, f->comp(c), host + (int64_t)c * nk, nk);
 }
 
 }  // namespace xcal

@@ -204,6 +204,8 @@ struct xcal_mesh {
   // device numbering: cperm/fperm map reference cell/face ids to device ids,
   // nzperm maps reference CSR slots to device slots
   std::vector<int32_t> cperm, fperm, nzperm;
+  xcal::DBuf<int32_t> cperm_d, fperm_d;  // the same on the device, for field transfers
+  mutable xcal::DBuf<double> stage;      // their buffer, of the largest field moved so far
   // CSR pattern in the reference's numbering (host only)
   std::vector<int32_t> h_rowptr, h_colval;
   // device matrix storage (sliced ELL): entries of row c at
@@ -437,11 +439,12 @@ void simple_case_field(const xcal_simple* S, int which, int k, double* host);
 // the k-omega fields
 int64_t prepared_footprint(const PreparedMesh& P, bool turb = false);
 int64_t prepared_cells(const PreparedMesh& P);
-void upload_permuted(const xcal_mesh* m, const std::vector<int32_t>& perm, double* dev,
-                     const double* host, int64_t len);
-// host[i] = dev[perm[i]] for i < len; dev holds dev_len entries (default len)
-void download_permuted(const xcal_mesh* m, const std::vector<int32_t>& perm, const double* dev,
-                       double* host, int64_t len, int64_t dev_len = -1);
+// dev[perm[i]] = host[i] and host[i] = dev[perm[i]], i < len, renumbered on
+// the device (perm is a device array: cperm_d, fperm_d or a part of one)
+void upload_permuted(const xcal_mesh* m, const int32_t* perm, double* dev, const double* host,
+                     int64_t len);
+void download_permuted(const xcal_mesh* m, const int32_t* perm, const double* dev, double* host,
+                       int64_t len);
 TermsK make_terms(const xcal_term* terms, int n);
 BCsK make_bcs(const xcal_mesh* m, const xcal_bc* bcs, int n);
 xcal_field* check_field(const xcal_field* f, const xcal_mesh* m, int kind, const char* what);
