@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "solver_common.h"
+#include "sweep_lean.h"
 #include "sweep_pipe.h"
 
 namespace xcal {
@@ -540,6 +541,7 @@ struct BSolver {
   MatKT<T> A;
   const T *Sj, *rD, *Lnz, *Unz, *Db;
   const T* Lrd;  // 1/D per packed lower entry (pipelined sweeps)
+  const T *La, *Ua;  // lean sweeps: a_ij by position
   T* work;
   KS* ks;
   double* partial;  // nblk slots (also used for the ncase sweep slots)
@@ -603,6 +605,8 @@ static BSolver<double> batch_solver(xcal_eqn* e) {
   S.Unz = e->Unz.p;
   S.Db = e->Db.p;
   S.Lrd = e->Lrd.p;
+  S.La = e->La.p;
+  S.Ua = e->Ua.p;
   S.work = e->work.p;
   S.ks = (KS*)e->kstate.p;
   S.partial = e->kpart.p;
@@ -631,6 +635,12 @@ static BSolver<float> batch_solver32(xcal_eqn* e) {
     tofloat(n, e->Db.p, e->Db32.p);
     tofloat(e->Lnz.n, e->Lnz.p, e->Lnz32.p);
     tofloat(e->Unz.n, e->Unz.p, e->Unz32.p);
+    if (m->lean) {
+      if (e->La32.n != e->La.n) e->La32.alloc(e->La.n);
+      if (e->Ua32.n != e->Ua.n) e->Ua32.alloc(e->Ua.n);
+      tofloat(e->La.n, e->La.p, e->La32.p);
+      tofloat(e->Ua.n, e->Ua.p, e->Ua32.p);
+    }
     if (m->pipe_wf > 0) {
       if (e->Lrd32.n != e->Lrd.n) e->Lrd32.alloc(e->Lrd.n);
       tofloat(e->Lrd.n, e->Lrd.p, e->Lrd32.p);
@@ -652,6 +662,8 @@ static BSolver<float> batch_solver32(xcal_eqn* e) {
   S.Unz = e->Unz32.p;
   S.Db = e->Db32.p;
   S.Lrd = e->Lrd32.p;
+  S.La = e->La32.p;
+  S.Ua = e->Ua32.p;
   S.work = e->work32.p;
   S.ks = (KS*)e->kstate.p;
   S.partial = e->kpart.p;
@@ -749,7 +761,13 @@ static void bsweep_fwd(const BSolver<T>& S, const FwdK<T>& W, const KS* ks, int 
   if (UPD && m->pipe_wf > 0)
     hipLaunchKernelGGL(kb_cg_xr<T>, dim3(S.nblk), dim3(kBlock), 0, S.s, S.B, W.x, W.p, W.r, W.q,
                        ks);
-  if (m->pipe_wf > 0)
+  if (m->lean && rw == 1)  // one row per thread: the lean body
+    with_lean_form(m->lean_f, [&](auto Wc, auto R) {
+      hipLaunchKernelGGL((k_fwd_lean<T, decltype(Wc)::value, decltype(R)::value>),
+                         dim3(S.ncase), dim3(kLeanBlock), 0, S.s, lean_k(m, m->lean_f), S.La, W.rD,
+                         UPD ? (const T*)W.r : W.u, W.posb, W.Yb, ks);
+    });
+  else if (m->pipe_wf > 0)
     with_pipe_form(m->pipe_wf, m->pipe_far_f, [&](auto WK, auto FAR) {
       with_pipe_rows(rw, [&](auto RW) {
         pipe(kb_fwd_pipe<UPD, decltype(FAR)::value, T, decltype(WK)::value, decltype(RW)::value>);
@@ -767,7 +785,12 @@ static void bsweep_bwd(const BSolver<T>& S, const BwdK<T>& W, const KS* ks, int 
     hipLaunchKernelGGL(kern, dim3(S.ncase), dim3(kPipeBlock / rw), 0, S.s, W, m->Upos.p,
                        m->lev_ptr_b_d.p, m->lmeta_b_d.p, m->case_lev_b_d.p, ks);
   };
-  if (m->pipe_wb > 0)
+  if (m->lean && rw == 1)
+    with_lean_form(m->lean_b, [&](auto Wc, auto R) {
+      hipLaunchKernelGGL((k_bwd_lean<DOT, T, decltype(Wc)::value, decltype(R)::value>),
+                         dim3(S.ncase), dim3(kLeanBlock), 0, S.s, lean_k(m, m->lean_b), S.Ua, W, ks);
+    });
+  else if (m->pipe_wb > 0)
     with_pipe_form(m->pipe_wb, m->pipe_far_b, [&](auto WK, auto FAR) {
       with_pipe_rows(rw, [&](auto RW) {
         pipe(kb_bwd_pipe<DOT, decltype(FAR)::value, T, decltype(WK)::value, decltype(RW)::value>);
@@ -1254,6 +1277,14 @@ static void bir_solve(xcal_eqn* e, const xcal_solver_setup* st, int itmax, doubl
 void precond_update_batch(xcal_eqn* e) {
   const xcal_mesh* m = e->mesh;
   hipStream_t s = m->ctx->stream;
+  if (m->lean && m->pipe_rw_f <= 1) {  // one row per thread, or not tuned yet
+    with_lean_form(m->lean_f, [&](auto Wc, auto R) {
+      hipLaunchKernelGGL((k_diag_lean<decltype(Wc)::value, decltype(R)::value>),
+                         dim3(m->ncase), dim3(kLeanBlock), 0, s, lean_k(m, m->lean_f),
+                         (const double*)e->Lp.p, e->pD.p);
+    });
+    return;
+  }
   if (m->pipe_wf > 0) {
     const int64_t nl = m->Lslot.n;
     if (e->Lprod.n != nl) e->Lprod.alloc(nl);

@@ -14,6 +14,7 @@
 
 #include "device_common.h"
 #include "sweep_cone.h"
+#include "sweep_lean.h"
 #include "sweep_pipe.h"
 
 namespace xcal {
@@ -257,6 +258,41 @@ void precond_update(xcal_eqn* e, int precon) {
                        e->nzval.p, e->pD.p);
     launch_check();
     const MatK A = matk(m, e->nzval.p);
+    // lean sweeps: products for the diagonal update, then the factors by position
+    auto lean_products = [&] {
+      const int64_t k = m->lean_f.slot.n;
+      if (e->Lp.n != k) e->Lp.alloc(k);
+      hipLaunchKernelGGL(k_lower_products, dim3(grid_for(k)), dim3(kBlock), 0, s, k,
+                         m->lean_f.slot.p, m->trans.p, e->nzval.p, e->Lp.p);
+    };
+    auto lean_factors = [&] {
+      auto fill = [&](DBuf<double>& a, const DBuf<int32_t>& slot) {
+        if (a.n != slot.n) a.alloc(slot.n);
+        hipLaunchKernelGGL(k_gather_slots, dim3(grid_for(slot.n)), dim3(kBlock), 0, s, slot.n,
+                           slot.p, e->nzval.p, a.p);
+      };
+      fill(e->La, m->lean_f.slot);
+      fill(e->Ua, m->lean_b.slot);
+    };
+    if (m->lean && !m->batch) {
+      lean_products();
+      with_lean_form(m->lean_f, [&](auto Wc, auto R) {
+        hipLaunchKernelGGL((k_diag_lean<decltype(Wc)::value, decltype(R)::value>), dim3(1),
+                           dim3(kLeanBlock), 0, s, lean_k(m, m->lean_f), (const double*)e->Lp.p,
+                           e->pD.p);
+      });
+      hipLaunchKernelGGL(k_recip, dim3(grid_for(n)), dim3(kBlock), 0, s, n, e->pD.p, e->prD.p);
+      lean_factors();
+      if (e->Db.n != n) e->Db.alloc(n);
+      hipLaunchKernelGGL(k_gather_rows, dim3(grid_for(n)), dim3(kBlock), 0, s, n, m->lev_rows_b.p,
+                         e->pD.p, e->Db.p);
+      launch_check();
+      return;
+    }
+    if (m->lean) {
+      lean_products();
+      lean_factors();
+    }
     if (!m->batch && m->pipe_runs) {  // a_ij a_ji per packed lower entry
       if (e->Lprod.n != m->Lslot.n) e->Lprod.alloc(m->Lslot.n);
       hipLaunchKernelGGL(k_lower_products, dim3(grid_for(m->Lslot.n)), dim3(kBlock), 0, s,

@@ -30,6 +30,7 @@
 
 #include "solver_common.h"
 #include "sweep_cone.h"
+#include "sweep_lean.h"
 #include "sweep_pipe.h"
 
 namespace xcal {
@@ -565,6 +566,7 @@ struct Solver {
   const T *D, *rD, *Sj;  // DILU D and 1/D; Jacobi 1/|a_ii|
   const T *Lnz, *Unz, *Db;  // packed DILU factors, D in backward-level order
   const T* Lrd;             // 1/D per packed lower entry (pipelined runs)
+  const T *La, *Ua;         // lean sweeps: a_ij by position
   // cone form: a_ij and 1/D_j per forward entry, 1/D per forward position,
   // a_ij per backward entry, D per backward position
   const T *cfa, *cfr, *cfd, *cba, *cbd;
@@ -625,6 +627,8 @@ static Solver<double> make_solver(xcal_eqn* e) {
   S.Unz = e->Unz.p;
   S.Db = e->Db.p;
   S.Lrd = e->Lrd.p;
+  S.La = e->La.p;
+  S.Ua = e->Ua.p;
   S.cfa = e->cfa.p;
   S.cfr = e->cfr.p;
   S.cfd = e->cfd.p;
@@ -674,7 +678,15 @@ static Solver<float> make_solver32(xcal_eqn* e) {
     hipLaunchKernelGGL(k_to_float, dim3(grid_for(n)), dim3(kBlock), 0, s, n, e->pD.p, e->pD32.p);
     hipLaunchKernelGGL(k_to_float, dim3(grid_for(n)), dim3(kBlock), 0, s, n, e->prD.p, e->prD32.p);
   }
-  if (e->precon == XCAL_PRECON_DILU && !m->cone) {  // the level sweeps' packed factors
+  if (e->precon == XCAL_PRECON_DILU && m->lean) {  // the lean sweeps' factors
+    auto cvt = [&](DBuf<float>& d, const DBuf<double>& a) {
+      if (d.n != a.n) d.alloc(a.n);
+      hipLaunchKernelGGL(k_to_float, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a.n, a.p, d.p);
+    };
+    cvt(e->La32, e->La);
+    cvt(e->Ua32, e->Ua);
+    cvt(e->Db32, e->Db);
+  } else if (e->precon == XCAL_PRECON_DILU && !m->cone) {  // the level sweeps' packed factors
     if (e->Lnz32.n != e->Lnz.n) e->Lnz32.alloc(e->Lnz.n);
     if (e->Unz32.n != e->Unz.n) e->Unz32.alloc(e->Unz.n);
     if (e->Db32.n != n) e->Db32.alloc(n);
@@ -709,6 +721,8 @@ static Solver<float> make_solver32(xcal_eqn* e) {
   S.Unz = e->Unz32.p;
   S.Db = e->Db32.p;
   S.Lrd = e->Lrd32.p;
+  S.La = e->La32.p;
+  S.Ua = e->Ua32.p;
   S.cfa = e->cfa32.p;
   S.cfr = e->cfa32.p;  // unused by the folded FP32 forward cone sweep
   S.cfd = e->cfa32.p;  // likewise
@@ -805,6 +819,18 @@ static void sweep_fwd(const Solver<T>& S, const FwdK<T>& W, const KStep* K = nul
     });
     return;
   }
+  if (m->lean) {
+    if (UPD)
+      hipLaunchKernelGGL(k_cg_xr<T>, dim3(grid_for(m->n)), dim3(kBlock), 0, S.s, 0, (int32_t)m->n,
+                         W.x, W.p, W.r, W.q, W.ks);
+    with_lean_form(m->lean_f, [&](auto Wc, auto R) {
+      constexpr int w = decltype(Wc)::value, ring = decltype(R)::value;
+      hipLaunchKernelGGL((k_fwd_lean<T, w, ring>), dim3(1), dim3(kLeanBlock), 0, S.s,
+                         lean_k(m, m->lean_f), S.La, W.rD, UPD ? (const T*)W.r : W.u, W.posb, W.Yb,
+                         W.ks);
+    });
+    return;
+  }
   for (const SweepStep& st : m->plan_f) {
     if (st.grid == 1 && st.pipe > 0) {
       if (UPD)
@@ -856,6 +882,23 @@ static void sweep_bwd(const Solver<T>& S, const BwdK<T>& W) {
                              S.cba, S.cbd, W, W.Yb);
       }
     });
+    return;
+  }
+  if (m->lean) {
+    with_lean_form(m->lean_b, [&](auto Wc, auto R) {
+      constexpr int w = decltype(Wc)::value, ring = decltype(R)::value;
+      const LeanK K = lean_k(m, m->lean_b);
+      if (m->lean_dots)
+        hipLaunchKernelGGL((k_bwd_lean<DOT, T, w, ring>), dim3(1), dim3(kLeanBlock), 0, S.s, K,
+                           S.Ua, W, W.ks);
+      else
+        hipLaunchKernelGGL((k_bwd_lean<0, T, w, ring>), dim3(1), dim3(kLeanBlock), 0, S.s, K, S.Ua,
+                           W, W.ks);
+    });
+    if (DOT != 0 && !m->lean_dots)
+      hipLaunchKernelGGL((k_plan_dots<DOT, T>), dim3(m->sweep_slots), dim3(kBlock), 0, S.s,
+                         m->dot_tab.p, W.rows, m->lev_ptr_b_d.p, W.dv, (const T*)W.Z, W.partial,
+                         W.ks);
     return;
   }
   for (const SweepStep& st : m->plan_b) {
@@ -925,6 +968,8 @@ void precond_apply_staged(xcal_eqn* e, const double* r, double* z, double* Y, do
   S.Unz = e->Unz.p;
   S.Db = e->Db.p;
   S.Lrd = e->Lrd.p;
+  S.La = e->La.p;
+  S.Ua = e->Ua.p;
   S.cfa = e->cfa.p;
   S.cfr = e->cfr.p;
   S.cfd = e->cfd.p;

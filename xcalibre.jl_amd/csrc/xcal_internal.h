@@ -95,6 +95,13 @@ constexpr int kConeMinBlock = 64;          // smallest block of a band
 constexpr int kConeBandBlocks = 512;       // blocks a band's block size aims at
 constexpr double kConeBandRatio = 4.0;     // most cone positions per row of a band
 
+// Lean one-workgroup sweeps (sweep_lean.h): threads, prefetch depth (and
+// padding of a case's steps), longest LDS ring, widest row.
+constexpr int kLeanBlock = 256;
+constexpr int kLeanDepth = 8;
+constexpr int kLeanRing = 8192;
+constexpr int kLeanWidth = 3;
+
 // Cut c_x (x = 0..8) of a level of cnt rows into eighths at 64-row
 // boundaries; eighth x is worked by the workgroups on XCD x.
 inline int64_t eighth_cut(int64_t cnt, int x) { return x >= 8 ? cnt : cnt * x / 8 / 64 * 64; }
@@ -289,6 +296,18 @@ struct xcal_mesh {
   int cone_nblk = 0, cone_rows = 0;  // forward blocks, rows per block
   bool cone_deep = false;            // deep prefetch (XCAL_CONE_DEEP=1 at creation)
   Cone cone_f, cone_b;
+  // Lean sweeps (sweep_lean.h), when both directions have them: a single
+  // mesh's whole sweep or every case of a batch, one workgroup each
+  struct Lean {
+    int w = 0, ring = 0;                 // entries per row, LDS ring
+    xcal::DBuf<int2> steps;              // first position, rows
+    xcal::DBuf<int32_t> cstep, slot;     // per case: first step; nz slot per entry (-1: none)
+    xcal::DBuf<uint32_t> idx;            // ring slots, two per word
+  };
+  bool lean = false;
+  bool lean_dots = false;  // the backward sweep sums its dots itself (k_plan_dots otherwise)
+  Lean lean_f, lean_b;
+  xcal::DBuf<int4> dot_tab;  // k_plan_dots: one entry per backward partial slot
   int small_level = 0;
   std::vector<SweepStep> plan_f, plan_b;
   int sweep_slots = 0;  // partial-sum slots used by one backward sweep
@@ -321,6 +340,8 @@ struct xcal_eqn {
   xcal::DBuf<double> Lnz, Unz, Db;  // packed factor values; D in backward-level order
   xcal::DBuf<double> Lrd;  // 1/D of each packed lower entry's column (0 on padding)
   xcal::DBuf<double> Lprod;  // a_ij a_ji of each packed lower entry (DILU diagonal update)
+  xcal::DBuf<double> La, Ua, Lp;  // lean sweeps: a_ij of both, a_ij a_ji of the lower entries
+  xcal::DBuf<float> La32, Ua32;
   // cone form: a_ij and 1/D_j per forward cone entry, a_ij per backward cone
   // entry, D per backward cone position
   xcal::DBuf<double> cfa, cfr, cfd, cba, cbd;
