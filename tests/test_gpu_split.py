@@ -1,0 +1,95 @@
+"""Split-preconditioned CG on cone meshes (two sweeps per iteration, no matrix
+product) against the classical iteration (XCAL_NO_SPLIT=1 at mesh creation).
+
+In exact arithmetic the two have the same iterates and stopping norm.  Each
+solve stops at a relative residual of 1e-6, so the first solve's solution is
+1e-6 times the conditioning left by DILU from the exact one and rounding that
+CG carries through some hundred iterations shows up below that (measured
+1.4e-5 from exact, 1.3e-7 between the forms).  The second solve takes the
+first's 1e-6 to 1e-12; the conditioning is some 1e1 to 1e2 there (1.4e-5 over
+1e-6), so the solutions may differ by 1e-10, and are compared at 1e-9
+(measured 1.4e-11 and below).  Matrices it does not apply to -- not symmetric,
+or changed since the preconditioner was made -- take the classical iteration
+and give its result bit for bit."""
+import numpy as np
+import pytest
+
+from conftest import rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(x):
+    return x.hip.Context(0)
+
+
+def _mesh(x, name):
+    if name == "quad":
+        return x.mesh.cavity2d(259)  # 67 081 cells, two entries per triangle, bands
+    nx, ny, nz, perm = {"random": (41, 40, 43, 7), "natural": (41, 40, 43, 0),
+                        "flat": (9, 90, 89, 7)}[name]
+    return x.mesh.box3d(nx, ny, nz, jitter=0.1, seed_perm=perm)
+
+
+def _solve(x, A, ctx, mesh, monkeypatch, off, prec="PREC_FP64", itmax=600, asym=False,
+           stale=False):
+    H = x.hip
+    if off:
+        monkeypatch.setenv("XCAL_NO_SPLIT", "1")
+    dm = H.DeviceMesh(ctx, mesh)
+    monkeypatch.delenv("XCAL_NO_SPLIT", raising=False)
+    assert dm.cone_form()[0] > 0
+    rng = np.random.default_rng(8)
+    g = H.Field(dm, A.FACE_SCALAR).upload(0.5 + rng.random(mesh.n_faces))
+    md = H.Field(dm, A.FACE_SCALAR).upload(1e-3 * rng.standard_normal(mesh.n_faces))
+    s = H.Field(dm, A.CELL_SCALAR).upload(rng.standard_normal(mesh.n_cells))
+    phi = H.Field(dm, A.CELL_SCALAR).upload(rng.standard_normal(mesh.n_cells))
+    eq = H.Equation(dm, False)
+    terms = [(A.LAPLACIAN_LINEAR, -1, g)] + ([(A.DIV_UPWIND, 1, md)] if asym else [])
+    bcs = A.bc_array([(A.BC_DIRICHLET if i == 0 else A.BC_ZEROGRADIENT, i, 0.0)
+                      for i in range(len(mesh.patch_names))])
+    eq.discretise(terms, [(s, 1)])
+    eq.apply_bcs(terms, bcs, phi)
+    eq.precond_update(A.PRECON_DILU)
+    if stale:
+        eq.set_reference(0.25)
+    setup = A.SolverSetupC(A.SOLVER_CG, A.PRECON_DILU, getattr(A, prec), itmax, 1e-7, 1.0, 1e-14,
+                           1e-10, 1e-6, 0, 0.0)
+    out = []
+    for _ in range(2):  # the second solve starts from the first one's result
+        n, res, rc = eq.solve(setup, phi)
+        out.append((n, rc, phi.download()))
+    return out
+
+
+@pytest.mark.parametrize("name", ["random", "natural", "flat", "quad"])
+@pytest.mark.parametrize("prec", ["PREC_FP64", "PREC_FP32_IR"])
+def test_split_cg_equals_classical_cg(x, A, ctx, monkeypatch, name, prec):
+    mesh = _mesh(x, name)
+    a = _solve(x, A, ctx, mesh, monkeypatch, False, prec)
+    b = _solve(x, A, ctx, mesh, monkeypatch, True, prec)
+    for u, v in zip(a, b):
+        assert u[1] == v[1] == 0
+        assert abs(u[0] - v[0]) <= (2 if prec == "PREC_FP64" else 6), (u[0], v[0])
+    assert rel(a[1][2], b[1][2]) < 1e-9
+    assert not np.array_equal(a[0][2], b[0][2])  # the split form ran
+
+
+@pytest.mark.parametrize("kind", ["asym", "stale"])
+@pytest.mark.parametrize("name", ["random", "natural"])
+def test_split_cg_leaves_other_systems_alone(x, A, ctx, monkeypatch, name, kind):
+    mesh = _mesh(x, name)
+    for u, v in zip(_solve(x, A, ctx, mesh, monkeypatch, False, itmax=40, **{kind: True}),
+                    _solve(x, A, ctx, mesh, monkeypatch, True, itmax=40, **{kind: True})):
+        assert u[:2] == v[:2] and np.array_equal(u[2], v[2])
+
+
+@pytest.mark.parametrize("itmax", [1, 2, 7])
+def test_split_cg_stops_at_itmax(x, A, ctx, monkeypatch, itmax):
+    mesh = _mesh(x, "random")
+    a = _solve(x, A, ctx, mesh, monkeypatch, False, itmax=itmax)
+    b = _solve(x, A, ctx, mesh, monkeypatch, True, itmax=itmax)
+    for u, v in zip(a, b):
+        assert u[0] == v[0] == itmax and u[1] == v[1] == 1
+        assert rel(u[2], v[2]) < 1e-12  # a few iterations' rounding

@@ -153,6 +153,7 @@ __global__ void k_set_reference(const int32_t* diag, double* nzval, double* b, d
 void discretise(xcal_eqn* e, const TermsK& t, const SourcesK& s, const xcal_field* prev, double dt) {
   xcal_mesh* m = e->mesh;
   e->cn = t.cn_first != 0;
+  e->nz_gen++;
   MeshK mk = meshk(m);
   double* nz = e->vector ? e->nzval0.p : e->nzval.p;
   const double* px = prev ? prev->comp(0) : nullptr;
@@ -175,6 +176,7 @@ void apply_bcs(xcal_eqn* e, const TermsK& t, const BCsK& b, const xcal_field* ph
   const double* py = phi->ncomp == 3 ? phi->comp(1) : px;
   const double* pz = phi->ncomp == 3 ? phi->comp(2) : px;
   double* bb = e->vector ? e->bc(comp) : e->bc(0);
+  e->nz_gen++;
   hipLaunchKernelGGL(k_apply_bcs, dim3(grid_for(m->nbcell)), dim3(kBlock), 0, m->ctx->stream,
                      meshk(m), t, b, e->vector ? comp : -1, px, py, pz, e->nzval.p, bb);
   XCAL_HIP(hipGetLastError());
@@ -182,6 +184,7 @@ void apply_bcs(xcal_eqn* e, const TermsK& t, const BCsK& b, const xcal_field* ph
 
 void relax_diagdom(xcal_eqn* e, const double* field, double* b, double alpha) {
   xcal_mesh* m = e->mesh;
+  e->nz_gen++;
   hipLaunchKernelGGL(k_relax_diagdom, dim3(grid_for(m->n)), dim3(kBlock), 0, m->ctx->stream, m->n,
                      m->rbeg.p, m->rend.p, m->diag.p, e->nzval.p, b, field, alpha);
   XCAL_HIP(hipGetLastError());
@@ -189,6 +192,7 @@ void relax_diagdom(xcal_eqn* e, const double* field, double* b, double alpha) {
 
 void set_reference(xcal_eqn* e, double pref, int64_t cell) {
   xcal_mesh* m = e->mesh;
+  e->nz_gen++;
   hipLaunchKernelGGL(k_set_reference, dim3(1), dim3(1), 0, m->ctx->stream, m->diag.p, e->nzval.p,
                      e->bc(0), pref, cell);
   XCAL_HIP(hipGetLastError());
@@ -303,6 +307,7 @@ int xcal_update_equation(xcal_eqn* e) {
   return guarded([&] {
     XCAL_CHECK(e && e->vector, "update_equation! applies to vector equations");
     copy_nz(e->mesh, e->nzval.p, e->nzval0.p);
+    e->nz_gen++;
     return 0;
   });
 }

@@ -349,7 +349,10 @@ static bool build_band(int S, double ratio, bool lower, const std::vector<int32_
 // covering only the band's rows: a band's block size is the power of two
 // (kConeMinBlock..S) that gives about kConeBandBlocks blocks, so a launch
 // still fills the chip, doubled while its cone positions exceed
-// kConeBandRatio times its rows (larger blocks recompute fewer rows).  A
+// kConeBandRatio times its rows (larger blocks recompute fewer rows; fewer,
+// wider bands pay for more recomputed rows: PISO on 308k naturally numbered
+// cells 160, 141, 135, 127, 125 ms at ratios 2, 3, 4, 6, 8, 85k cells 45.9,
+// 40.3, 39.2, 36.3, 36.1, and 8 holds a third more positions than 6).  A
 // band starts at twice the previous band's width (the levels left, for the
 // first) and halves when no block size fits.  False
 // when a band of kConeMinBand levels does not fit, the sweep needs more than
@@ -399,6 +402,51 @@ static bool build_cone(int64_t n, int S, bool lower, const std::vector<int32_t>&
   if (C.wk == 0 || C.lidx.empty()) return false;  // masked loads read entry 0
   C.wk = C.wk <= 2 ? 2 : C.wk <= 4 ? 4 : C.wk <= 6 ? 6 : 8;
   return true;
+}
+
+// Tables of the split CG's sweeps from a cone's (sweep_split.h): per position
+// its row and six 16-bit slots (kConeMax: none), a step's entries in pairs
+// (pair j of rows [0, pcnt[j]), which have more than 2 j entries), steps padded
+// per block to whole groups with repeats of the last row.  False where a row
+// has more than six entries or an index would pass 32-bit byte offsets.
+static bool build_split(const ConeHost& H, std::vector<int32_t>& step, std::vector<int32_t>& blk,
+                        std::vector<int4>& rec, std::vector<int32_t>& pslot) {
+  if (H.wk > 6 || H.crow.size() >= (1u << 28)) return false;
+  rec.assign(H.crow.size(), int4{0, 0, 0, 0});
+  pslot.assign(2, -1);
+  blk.assign(1, 0);
+  for (size_t b = 0; b + 1 < H.blk.size(); ++b) {
+    int32_t last[8] = {};
+    for (int32_t s = H.blk[b]; s < H.blk[b + 1]; ++s) {
+      const int32_t* t = &H.steps[(size_t)s * kConeTab];
+      const int32_t r0 = t[0], cnt = t[1], *eoff = t + 2, *ecnt = t + 10;
+      int32_t out[8] = {r0, cnt};
+      for (int32_t q = 0; q < cnt; ++q) {
+        uint32_t w[3] = {0, 0, 0};
+        for (int k = 0; k < 6; ++k)
+          w[k / 2] |= (uint32_t)(q < ecnt[k] ? H.lidx[eoff[k] + q] : kConeMax) << 16 * (k % 2);
+        rec[r0 + q] = int4{H.crow[r0 + q], (int)w[0], (int)w[1], (int)w[2]};
+      }
+      for (int j = 0; j < 3; ++j) {
+        out[2 + j] = (int32_t)(pslot.size() / 2);
+        out[5 + j] = ecnt[2 * j];
+        for (int32_t q = 0; q < ecnt[2 * j]; ++q)
+          for (int k = 2 * j; k < 2 * j + 2; ++k)
+            pslot.push_back(q < ecnt[k] ? H.slot[eoff[k] + q] : -1);
+      }
+      step.insert(step.end(), out, out + 8);
+      last[0] = r0 + cnt - 1;  // the step's last row alone, in no dot product
+      for (int j = 0; j < 3; ++j) {
+        const bool has = out[5 + j] == cnt;
+        last[2 + j] = has ? out[2 + j] + cnt - 1 : 0;
+        last[5 + j] = has ? 1 : 0;
+      }
+    }
+    while ((step.size() / 8 - blk.back()) % kSplitDepth != 0)
+      step.insert(step.end(), last, last + 8);
+    blk.push_back((int32_t)(step.size() / 8));
+  }
+  return pslot.size() / 2 < (1u << 28);
 }
 
 // DILU levels, renumbering, sliced-ELL slots and packed factors.
@@ -1193,6 +1241,20 @@ static xcal_mesh* upload_mesh(xcal_ctx* ctx, HostMesh& M) {
     up(m->cone_b, M.cone_b);
     upload(m->cone_own, M.cone_f.own, bytes);
     upload(m->cone_ownp, M.cone_f.ownp, bytes);
+    const char* nosplit = std::getenv("XCAL_NO_SPLIT");
+    if (!(nosplit && *nosplit == '1') && M.n < (1 << 28)) {
+      std::vector<int32_t> st[2], bl[2], ps[2];
+      std::vector<int4> rc[2];
+      m->split = build_split(M.cone_f, st[0], bl[0], rc[0], ps[0]) &&
+                 build_split(M.cone_b, st[1], bl[1], rc[1], ps[1]);
+      for (int d = 0; m->split && d < 2; ++d) {
+        xcal_mesh::Cone& D = d ? m->cone_b : m->cone_f;
+        upload(D.step2, st[d], bytes);
+        upload(D.blk2, bl[d], bytes);
+        upload(D.rec, rc[d], bytes);
+        upload(D.pslot, ps[d], bytes);
+      }
+    }
     m->cone = true;
     m->cone_nblk = m->cone_f.nblk();
     m->cone_rows = M.cone_rows;

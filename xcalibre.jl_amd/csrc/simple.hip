@@ -384,6 +384,7 @@ int run_impl(xcal_simple* S, int32_t iterations, std::vector<double>& R, std::ve
       for (int c = 0; c < (is3d ? 3 : 2); ++c) {
         mark(2);
         copy_nz(m, Ue->nzval.p, Ue->nzval0.p);  // update_equation!
+        Ue->nz_gen++;
         apply_bcs(Ue, UT, S->bU, S->U, c);
         relax_diagdom(Ue, S->U->comp(c), Ue->bc(c), cfg.U.relax);
         if (c == 0) precond_update(Ue, cfg.U.precon);

@@ -31,6 +31,7 @@
 #include "solver_common.h"
 #include "sweep_cone.h"
 #include "sweep_lean.h"
+#include "sweep_split.h"
 #include "sweep_pipe.h"
 
 namespace xcal {
@@ -120,8 +121,6 @@ __global__ void __launch_bounds__(kBlock)
 // grid is a multiple of 8, so row block b is handled on the XCD of the SpMV
 // workgroup that reads it.  The rows' loads are issued before the
 // reduction, which they do not depend on.
-constexpr int kPFinU = 4;
-inline int pfin_grid(int nblk) { return ((nblk + kPFinU - 1) / kPFinU + 7) / 8 * 8; }
 template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_cg_p_fin(MatKT<T> A, int nblk, const T* __restrict__ z, const T* __restrict__ pold,
@@ -424,6 +423,33 @@ __global__ void __launch_bounds__(kBlock)
   if (i < n) b[i] = (float)(a[i] * rd[i]);
 }
 
+// split CG factors: nz of each entry of the pairs (0 where there is none),
+// and out[p] = v of cone position p's row
+__global__ void __launch_bounds__(kBlock)
+    k_split_pairs(int64_t n, const int32_t* __restrict__ slot, const double* __restrict__ nz,
+                  double* __restrict__ out) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e < n) out[e] = slot[e] >= 0 ? nz[slot[e]] : 0.0;
+}
+__global__ void __launch_bounds__(kBlock)
+    k_split_rows(int64_t total, const int32_t* __restrict__ crow, const double* __restrict__ v,
+                 double* __restrict__ out) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p < total) out[p] = v[crow[p] >= 0 ? crow[p] : ~crow[p]];
+}
+// (1/D, a_ii - D) per forward cone position
+__global__ void __launch_bounds__(kBlock)
+    k_split_scalars(int64_t total, const int32_t* __restrict__ crow,
+                    const int32_t* __restrict__ diag, const double* __restrict__ nz,
+                    const double* __restrict__ D, const double* __restrict__ rD,
+                    double* __restrict__ out) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= total) return;
+  const int32_t c = crow[p], i = c >= 0 ? c : ~c;
+  out[2 * p] = rD[i];
+  out[2 * p + 1] = nz[diag[i]] - D[i];
+}
+
 // b = 1 / a rounded to FP32
 __global__ void __launch_bounds__(kBlock)
     k_recip_float(int64_t n, const double* __restrict__ a, float* __restrict__ b) {
@@ -589,7 +615,9 @@ static void ensure_workspace(xcal_eqn* e, bool fp32) {
   const xcal_mesh* m = e->mesh;
   const int64_t n = m->n;
   const int64_t slots =
-      std::max<int64_t>(std::max<int64_t>(grid_for(n), m->nxblk), m->sweep_slots) + 8;
+      std::max<int64_t>(std::max<int64_t>(grid_for(n), m->nxblk),
+                        std::max<int64_t>(m->sweep_slots,
+                                          m->cone_nblk + pfin_grid(m->nxblk))) + 8;
   const bool grow = (e->work.n > 0 && e->work.n < 12 * n) ||
                     (e->kpart.n > 0 && e->kpart.n < 2 * slots) ||
                     (fp32 && e->work32.n > 0 && e->work32.n < 12 * n) ||
@@ -978,6 +1006,45 @@ void precond_apply_staged(xcal_eqn* e, const double* r, double* z, double* Y, do
   dilu_apply(S, r, z, Y, Yb);
 }
 
+// The split CG's factors (sweep_split.h), made at a solve from the
+// preconditioner's: only CG on a symmetric matrix uses them.
+template <class T>
+struct SplitFactors {
+  const T *a, *b, *f, *d;  // forward and backward pairs, (1/D, a_ii - D), 1/D
+};
+static SplitFactors<double> split_factors(xcal_eqn* e, double) {
+  const xcal_mesh* m = e->mesh;
+  const xcal_mesh::Cone &F = m->cone_f, &B = m->cone_b;
+  hipStream_t s = m->ctx->stream;
+  auto pairs = [&](DBuf<double>& v, const DBuf<int32_t>& slot) {
+    if (v.n != slot.n) v.alloc(slot.n);
+    hipLaunchKernelGGL(k_split_pairs, dim3(grid_for(slot.n)), dim3(kBlock), 0, s, slot.n, slot.p,
+                       (const double*)e->nzval.p, v.p);
+  };
+  pairs(e->spa, F.pslot);
+  pairs(e->spb, B.pslot);
+  if (e->spf.n != 2 * F.rows) e->spf.alloc(2 * F.rows);
+  if (e->spd.n != B.rows) e->spd.alloc(B.rows);
+  hipLaunchKernelGGL(k_split_scalars, dim3(grid_for(F.rows)), dim3(kBlock), 0, s, F.rows, F.crow.p,
+                     m->diag.p, (const double*)e->nzval.p, (const double*)e->pD.p,
+                     (const double*)e->prD.p, e->spf.p);
+  hipLaunchKernelGGL(k_split_rows, dim3(grid_for(B.rows)), dim3(kBlock), 0, s, B.rows, B.crow.p,
+                     (const double*)e->prD.p, e->spd.p);
+  XCAL_HIP(hipGetLastError());
+  return {e->spa.p, e->spb.p, e->spf.p, e->spd.p};
+}
+static SplitFactors<float> split_factors(xcal_eqn* e, float) {
+  split_factors(e, 0.0);
+  hipStream_t s = e->mesh->ctx->stream;
+  auto cvt = [&](DBuf<float>& d, const DBuf<double>& a) {
+    if (d.n != a.n) d.alloc(a.n);
+    hipLaunchKernelGGL(k_to_float, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a.n, a.p, d.p);
+    return (const float*)d.p;
+  };
+  return {cvt(e->spa32, e->spa), cvt(e->spb32, e->spb), cvt(e->spf32, e->spf),
+          cvt(e->spd32, e->spd)};
+}
+
 template <class T>
 static KS read_state(Solver<T>& S) {
   XCAL_HIP(hipMemcpyAsync(S.e->kstate_host, S.ks, sizeof(KS), hipMemcpyDeviceToHost, S.s));
@@ -1020,6 +1087,82 @@ static int run_batches(Solver<T>& S, int* pred, int tail, const std::function<vo
   return out.stop;
 }
 
+// Whether a CG solve takes the split form: cone mesh with its tables, FP64 or
+// refinement's FP32 sweeps, the preconditioner made from the matrix as it is
+// now, and the matrix symmetric to the last bit (one flag, read back).
+template <class T>
+static bool split_applies(Solver<T>& S, int precon) {
+  const xcal_eqn* e = S.e;
+  if (precon != XCAL_PRECON_DILU || !S.m->cone || !S.m->split || S.pc32 ||
+      e->precon_gen != e->nz_gen || e->asym.n < 1)
+    return false;
+  int32_t* flag = (int32_t*)(S.m->ctx->host_pinned + 60);
+  XCAL_HIP(hipMemcpyAsync(flag, e->asym.p, sizeof(int32_t), hipMemcpyDeviceToHost, S.s));
+  XCAL_HIP(hipStreamSynchronize(S.s));
+  return *flag == 0;
+}
+
+// The split form's iterations (sweep_split.h), from the residual r and x = 0
+// (pa = 0): three launches each, the scalar updates done by the next kernel.
+// Returns the final state.
+template <class T>
+static KS cg_split(Solver<T>& S, T* w) {
+  const int64_t n = S.n;
+  const xcal_mesh* m = S.m;
+  T *r = w, *x = w + n, *pa = w + 2 * n, *pb = w + 3 * n, *q = w + 4 * n, *t = w + 5 * n,
+    *rho = w + 6 * n;
+  const SplitFactors<T> f = split_factors(S.e, T(0));
+  const std::vector<int32_t>&bf = m->cone_f.band, &bb = m->cone_b.band;
+  T* wv = bf.size() > 2 ? w + 7 * n : nullptr;  // later bands read w as their halo
+  const int nf = m->cone_f.nblk(), vg = pfin_grid(S.gridA);
+  // the sweep's partials and the vector pass's, used in turn
+  double *p0 = S.partial, *p1 = S.partial + 2 * (int64_t)nf;
+  KS* cur = S.ks;
+  auto other = [&](KS* k) { return k == S.ks ? S.fks : S.ks; };
+  auto fwd = [&](auto start, const T* u, T* out) {
+    for (size_t k = 0; k + 1 < bf.size(); ++k)
+      hipLaunchKernelGGL((k_split_fwd<decltype(start)::value, T>), dim3(bf[k + 1] - bf[k]),
+                         dim3(kConeBlock), 0, S.s, split_k(m->cone_f, bf[k]), f.a, f.f, u,
+                         (const T*)t, out, wv, n, p0, (const KS*)cur);
+  };
+  fwd(std::true_type{}, (const T*)r, rho);
+  finalize_launch(S, nf, FIN_CG_INIT);
+  int parity = 0;
+  bool pend = false;
+  auto iteration = [&]() {
+    T* pold = parity ? pb : pa;
+    T* pnew = parity ? pa : pb;
+    parity ^= 1;
+    // the first band does the pending finalize, the others read its state
+    const KStep Kb{cur, other(cur), p1, vg, pend ? FIN_CG_ITER : FIN_NONE};
+    const KStep Kn = kstep_plain(other(cur));
+    timed(m->ctx, 2, [&] {
+      for (size_t k = 0; k + 1 < bb.size(); ++k)
+        hipLaunchKernelGGL(k_split_bwd<T>, dim3(bb[k + 1] - bb[k]), dim3(kConeBlock), 0, S.s,
+                           split_k(m->cone_b, bb[k]), f.b, f.d, (const T*)rho, (const T*)pold, pnew,
+                           t, n, k == 0 ? Kb : Kn);
+    });
+    cur = other(cur);
+    timed(m->ctx, 1, [&] { fwd(std::false_type{}, (const T*)pnew, q); });
+    const KStep Kv{cur, other(cur), p0, nf, FIN_CG_PAP};
+    cur = other(cur);
+    hipLaunchKernelGGL(k_split_vec<T>, dim3(vg), dim3(kBlock), 0, S.s, S.A, S.gridA, (const T*)t,
+                       (const T*)q, S.rD, x, rho, p1, Kv);
+    pend = true;
+  };
+  KS st = read_state(S);
+  if (st.stop == STOP_NONE)
+    run_batches(S, S.cg_batch, 4, iteration, st, [&] {
+      if (pend)  // an iteration leaves the state in S.ks, its last finalize pending
+        hipLaunchKernelGGL(k_finalize_to, dim3(1), dim3(kBlock), 0, S.s, (const double*)p1, vg,
+                           (const KS*)cur, S.ks, (int)FIN_CG_ITER);
+      pend = false;
+      cur = S.ks;
+    });
+  XCAL_HIP(hipGetLastError());
+  return st;
+}
+
 // Krylov.jl cg! with warm start x0 (solution = x0 + correction, written to
 // x0).  With x0 == NULL the start is zero and the solution is left in
 // *xsol (a workspace vector).  Returns 1 when itmax was reached.
@@ -1033,6 +1176,15 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
   init_state(S, itmax, atol, rtol);
   hipLaunchKernelGGL(k_start<T>, dim3(S.gridA), dim3(kBlock), 0, S.s, S.A, b, (const T*)x0, r, x, pa);
   const bool dilu = precon == XCAL_PRECON_DILU;
+  if (split_applies(S, precon)) {
+    const KS st = cg_split(S, w);
+    if (x0) hipLaunchKernelGGL(k_add, dim3(S.grid), dim3(kBlock), 0, S.s, n, (const double*)x,
+                               (double*)x0);
+    if (xsol) *xsol = x;
+    XCAL_HIP(hipGetLastError());
+    niter = st.iter;
+    return (st.stop == STOP_ITMAX || niter >= itmax) ? 1 : 0;
+  }
   const T* Sd = precon == XCAL_PRECON_JACOBI ? S.Sj : nullptr;
   const int sweep_slots = S.m->sweep_slots;
   if (dilu) {

@@ -201,6 +201,7 @@ void turb_wall_production(const xcal_mesh* m, const BCsK& bk, double nu, const d
 }
 void turb_omega_constrain(xcal_eqn* e, const BCsK& bw, double nu, const double* k) {
   const xcal_mesh* m = e->mesh;
+  e->nz_gen++;
   TLAUNCH(k_omega_constrain, m->nbcell, meshk(m), bw, wallk(nu), m->rbeg.p, m->rend.p, m->diag.p,
           k, e->nzval.p, e->bc(0));
 }

@@ -93,7 +93,8 @@ constexpr int kConeMinBand = 4;            // narrowest band of levels
 constexpr int kConeMaxBands = 128;         // most bands (launches) per sweep
 constexpr int kConeMinBlock = 64;          // smallest block of a band
 constexpr int kConeBandBlocks = 512;       // blocks a band's block size aims at
-constexpr double kConeBandRatio = 4.0;     // most cone positions per row of a band
+constexpr double kConeBandRatio = 6.0;     // most cone positions per row of a band
+constexpr int kSplitDepth = 4;  // steps in flight of the split CG's sweeps (and their padding)
 
 // Lean one-workgroup sweeps (sweep_lean.h): threads, prefetch depth (and
 // padding of a case's steps), longest LDS ring, widest row.
@@ -288,12 +289,18 @@ struct xcal_mesh {
     xcal::DBuf<int32_t> blk, base, steps, crow, slot, dep, hnum;
     xcal::DBuf<uint16_t> lidx;
     std::vector<int32_t> band;  // host: first block of each band (nbands + 1)
+    // the same steps with rows packed for the split CG (sweep_split.h): steps
+    // padded per block, one record per position, nz slots of the entry pairs
+    // (pair 0 is empty)
+    xcal::DBuf<int32_t> step2, blk2, pslot;
+    xcal::DBuf<int4> rec;
     int nblk() const { return band.empty() ? 0 : band.back(); }
   };
   // the forward sweep's block b owns rows cone_own[cone_ownp[b], cone_ownp[b+1])
   xcal::DBuf<int32_t> cone_own, cone_ownp;
   bool cone = false;
   int cone_nblk = 0, cone_rows = 0;  // forward blocks, rows per block
+  bool split = false;  // the split CG's tables were built (rows of at most 6 entries per triangle)
   bool cone_deep = false;            // deep prefetch (XCAL_CONE_DEEP=1 at creation)
   Cone cone_f, cone_b;
   // Lean sweeps (sweep_lean.h), when both directions have them: a single
@@ -340,6 +347,14 @@ struct xcal_eqn {
   xcal::DBuf<double> Lnz, Unz, Db;  // packed factor values; D in backward-level order
   xcal::DBuf<double> Lrd;  // 1/D of each packed lower entry's column (0 on padding)
   xcal::DBuf<double> Lprod;  // a_ij a_ji of each packed lower entry (DILU diagonal update)
+  // split CG on cone meshes: entry pairs of both sweeps, (1/D, a_ii - D) per
+  // forward and 1/D per backward position; asym != 0: A is not symmetric
+  xcal::DBuf<double> spa, spb, spf, spd;
+  xcal::DBuf<float> spa32, spb32, spf32, spd32;
+  xcal::DBuf<int32_t> asym;
+  // changes of nzval, and their count at the last preconditioner update: the
+  // split CG takes A's triangles from the preconditioner's factors
+  int64_t nz_gen = 0, precon_gen = -1;
   xcal::DBuf<double> La, Ua, Lp;  // lean sweeps: a_ij of both, a_ij a_ji of the lower entries
   xcal::DBuf<float> La32, Ua32;
   // cone form: a_ij and 1/D_j per forward cone entry, a_ij per backward cone
