@@ -431,11 +431,22 @@ __global__ void __launch_bounds__(kBlock)
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) out[e] = slot[e] >= 0 ? nz[slot[e]] : 0.0;
 }
+template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_split_rows(int64_t total, const int32_t* __restrict__ crow, const double* __restrict__ v,
-                 double* __restrict__ out) {
+    k_split_rows(int64_t total, const int32_t* __restrict__ crow, const T* __restrict__ v,
+                 T* __restrict__ out) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p < total) out[p] = v[crow[p] >= 0 ? crow[p] : ~crow[p]];
+}
+// the solution back in device order: x0 += x, or out = x
+template <bool ADD, class T>
+__global__ void __launch_bounds__(kBlock)
+    k_split_out(int64_t n, const int32_t* __restrict__ rows, const T* __restrict__ x,
+                T* __restrict__ out) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n) return;
+  const int32_t i = rows[p];
+  out[i] = ADD ? out[i] + x[p] : x[p];
 }
 // (1/D, a_ii - D) per forward cone position
 __global__ void __launch_bounds__(kBlock)
@@ -617,7 +628,7 @@ static void ensure_workspace(xcal_eqn* e, bool fp32) {
   const int64_t slots =
       std::max<int64_t>(std::max<int64_t>(grid_for(n), m->nxblk),
                         std::max<int64_t>(m->sweep_slots,
-                                          m->cone_nblk + pfin_grid(m->nxblk))) + 8;
+                                          m->cone_nblk + pfin_grid(grid_for(n)))) + 8;
   const bool grow = (e->work.n > 0 && e->work.n < 12 * n) ||
                     (e->kpart.n > 0 && e->kpart.n < 2 * slots) ||
                     (fp32 && e->work32.n > 0 && e->work32.n < 12 * n) ||
@@ -1028,7 +1039,7 @@ static SplitFactors<double> split_factors(xcal_eqn* e, double) {
   hipLaunchKernelGGL(k_split_scalars, dim3(grid_for(F.rows)), dim3(kBlock), 0, s, F.rows, F.crow.p,
                      m->diag.p, (const double*)e->nzval.p, (const double*)e->pD.p,
                      (const double*)e->prD.p, e->spf.p);
-  hipLaunchKernelGGL(k_split_rows, dim3(grid_for(B.rows)), dim3(kBlock), 0, s, B.rows, B.crow.p,
+  hipLaunchKernelGGL(k_split_rows<double>, dim3(grid_for(B.rows)), dim3(kBlock), 0, s, B.rows, B.crow.p,
                      (const double*)e->prD.p, e->spd.p);
   XCAL_HIP(hipGetLastError());
   return {e->spa.p, e->spb.p, e->spf.p, e->spd.p};
@@ -1104,17 +1115,24 @@ static bool split_applies(Solver<T>& S, int precon) {
 
 // The split form's iterations (sweep_split.h), from the residual r and x = 0
 // (pa = 0): three launches each, the scalar updates done by the next kernel.
-// Returns the final state.
+// Its vectors are in the split row order: r and 1/D are brought to it here,
+// x (in it) is left for k_split_out.  Returns the final state.
 template <class T>
 static KS cg_split(Solver<T>& S, T* w) {
   const int64_t n = S.n;
   const xcal_mesh* m = S.m;
   T *r = w, *x = w + n, *pa = w + 2 * n, *pb = w + 3 * n, *q = w + 4 * n, *t = w + 5 * n,
-    *rho = w + 6 * n;
+    *rho = w + 6 * n, *rD = w + 8 * n, *u0 = w + 9 * n;
   const SplitFactors<T> f = split_factors(S.e, T(0));
   const std::vector<int32_t>&bf = m->cone_f.band, &bb = m->cone_b.band;
   T* wv = bf.size() > 2 ? w + 7 * n : nullptr;  // later bands read w as their halo
-  const int nf = m->cone_f.nblk(), vg = pfin_grid(S.gridA);
+  const int nf = m->cone_f.nblk(), vg = pfin_grid((int)grid_for(n));
+  auto order = [&](const T* v, T* out) {
+    hipLaunchKernelGGL(k_split_rows<T>, dim3(grid_for(n)), dim3(kBlock), 0, S.s, n,
+                       m->split_rows.p, v, out);
+  };
+  order(r, u0);
+  order(S.rD, rD);
   // the sweep's partials and the vector pass's, used in turn
   double *p0 = S.partial, *p1 = S.partial + 2 * (int64_t)nf;
   KS* cur = S.ks;
@@ -1125,7 +1143,7 @@ static KS cg_split(Solver<T>& S, T* w) {
                          dim3(kConeBlock), 0, S.s, split_k(m->cone_f, bf[k]), f.a, f.f, u,
                          (const T*)t, out, wv, n, p0, (const KS*)cur);
   };
-  fwd(std::true_type{}, (const T*)r, rho);
+  fwd(std::true_type{}, (const T*)u0, rho);
   finalize_launch(S, nf, FIN_CG_INIT);
   int parity = 0;
   bool pend = false;
@@ -1146,8 +1164,8 @@ static KS cg_split(Solver<T>& S, T* w) {
     timed(m->ctx, 1, [&] { fwd(std::false_type{}, (const T*)pnew, q); });
     const KStep Kv{cur, other(cur), p0, nf, FIN_CG_PAP};
     cur = other(cur);
-    hipLaunchKernelGGL(k_split_vec<T>, dim3(vg), dim3(kBlock), 0, S.s, S.A, S.gridA, (const T*)t,
-                       (const T*)q, S.rD, x, rho, p1, Kv);
+    hipLaunchKernelGGL(k_split_vec<T>, dim3(vg), dim3(kBlock), 0, S.s, n, (const T*)t,
+                       (const T*)q, (const T*)rD, x, rho, p1, Kv);
     pend = true;
   };
   KS st = read_state(S);
@@ -1178,9 +1196,14 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
   const bool dilu = precon == XCAL_PRECON_DILU;
   if (split_applies(S, precon)) {
     const KS st = cg_split(S, w);
-    if (x0) hipLaunchKernelGGL(k_add, dim3(S.grid), dim3(kBlock), 0, S.s, n, (const double*)x,
-                               (double*)x0);
-    if (xsol) *xsol = x;
+    const int32_t* rows = S.m->split_rows.p;
+    if (x0) hipLaunchKernelGGL((k_split_out<true, T>), dim3(S.grid), dim3(kBlock), 0, S.s, n, rows,
+                               (const T*)x, x0);
+    if (xsol) {
+      hipLaunchKernelGGL((k_split_out<false, T>), dim3(S.grid), dim3(kBlock), 0, S.s, n, rows,
+                         (const T*)x, r);
+      *xsol = r;
+    }
     XCAL_HIP(hipGetLastError());
     niter = st.iter;
     return (st.stop == STOP_ITMAX || niter >= itmax) ? 1 : 0;

@@ -27,14 +27,20 @@
 // store's range check instead of a branch, which would end the loop's block
 // and with it exact waits.
 //
-// Measured on one MI355X, classical then split, per CG iteration: 1M-cell
-// random box 104 to 74 us (35 + 32 + 27 + 8 to 36 + 25 + 12; one box in
-// three ran the backward sweep at 48), 152k random box in FP32 57 to 36 us,
-// 308k natural box (bands) 530 to 420 us.  The backward sweep is bound by its
-// scattered rows (a backward level's rows lie in as many runs as there are
-// forward levels: two gathers and two stores of 8 bytes from 64 lines each),
-// the forward one by the step-to-step chain; 4 steps in flight, 6 and 5 were
-// no faster.
+// The vectors of a solve are in a row order of their own (split_rows): the
+// rows of a block together, there by forward, then by backward level.  A
+// backward step's rows then lie in one run per forward level inside 16 KB
+// instead of in a line each all over the level-major device order, and no
+// block's lines are another's.  The residual and 1/D are brought to it once a
+// solve and the solution back; the matrix, SpMV and every other solve keep
+// the device order (ordering that one by backward level cost SpMV 15%).
+//
+// Measured on one MI355X, per CG iteration: 1M-cell random box 104 us
+// classical (35 + 32 + 27 + 8), 87 split in device order (48 backward, 27
+// forward, 12 vectors), 66 in block order (28 + 26 + 11); 343k random box
+// 66, 43 and 40; 152k random box in FP32 57, 33 and 31; 308k natural box
+// (bands) 530 and 420.  Both sweeps are bound by the step-to-step chain and
+// the 1.75 n rows of the cones; 4 steps in flight, 6 and 5 were no faster.
 #pragma once
 
 #include "sweep_cone.h"
@@ -53,9 +59,8 @@ struct SplitK {
   const int32_t* step;  // 8 words per step: first position, rows, poff[3], pcnt[3]
   const int32_t* blk;   // first step of each block (whole groups of kSplitDepth)
   const int32_t* base;  // first position of each block
-  const int32_t* crow;  // device row of each position (halo staging)
   const int32_t* hnum;  // halo positions of each block
-  const int4* rec;      // per position: row (~row: another block's), slots 0-1, 2-3, 4-5
+  const int4* rec;      // per position: row (~row: another block's, or halo), slots 0-1, 2-3, 4-5
   int32_t blk0;
 };
 
@@ -87,7 +92,7 @@ struct SplitRec {
 
 // Walks block b's steps.  NS scalars per position at `sc`; g0 and, with NG = 2,
 // g1 are gathered from G0 and G1 by row; work(R, row, sum) returns the row's
-// value.  Halo values come from `halo`, in device order.
+// value.  Halo values come from `halo`.
 template <int NS, int NG, class T, class Work>
 __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ a,
                                   const T* __restrict__ sc, const T* __restrict__ halo,
@@ -97,7 +102,7 @@ __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ 
   constexpr int P = kSplitDepth, Q = kSplitGather;
   const int s0 = C.blk[b], ns = C.blk[b + 1] - s0;
   const int32_t base = C.base[b], nh = C.hnum[b];
-  for (int32_t p = threadIdx.x; p < nh; p += kConeBlock) v[p] = halo[~C.crow[base + p]];
+  for (int32_t p = threadIdx.x; p < nh; p += kConeBlock) v[p] = halo[~C.rec[base + p].x];
   if (threadIdx.x == 0) v[kConeMax] = T(0);
   __syncthreads();
   const auto* words = (const __attribute__((address_space(4))) int32_t*)(C.step + 8 * (int64_t)s0);
@@ -235,10 +240,10 @@ __global__ void __launch_bounds__(kConeBlock)
 }
 
 // Vectors: the pending ph.q/D finalize, then x += alpha t, rho -= alpha q and
-// the partials of rho.rho/D, over A's row blocks blockIdx.x + u gridDim.x.
+// the partials of rho.rho/D; kPFinU blocks of consecutive rows a workgroup.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_split_vec(MatKT<T> A, int nblk, const T* __restrict__ t, const T* __restrict__ q,
+    k_split_vec(int64_t n, const T* __restrict__ t, const T* __restrict__ q,
                 const T* __restrict__ rD, T* __restrict__ x, T* __restrict__ rho, double* partial,
                 KStep K) {
   __shared__ double lds[kBlock / 64];
@@ -246,10 +251,8 @@ __global__ void __launch_bounds__(kBlock)
   T xv[kPFinU], tv[kPFinU], rv[kPFinU], qv[kPFinU], dv[kPFinU];
 #pragma unroll
   for (int u = 0; u < kPFinU; ++u) {
-    const int b = (int)blockIdx.x + u * (int)gridDim.x;
-    const int bb = b < nblk ? b : 0;
-    const int64_t r = (int64_t)A.blk[2 * bb] + threadIdx.x;
-    i[u] = b < nblk && r < A.blk[2 * bb + 1] ? r : -1;
+    const int64_t r = (xcd_block() * kPFinU + u) * kBlock + threadIdx.x;
+    i[u] = r < n ? r : -1;
   }
 #pragma unroll
   for (int u = 0; u < kPFinU; ++u) {
@@ -277,7 +280,7 @@ __global__ void __launch_bounds__(kBlock)
 
 // Host: the kernel view of one direction's tables for the band from blk0.
 inline SplitK split_k(const xcal_mesh::Cone& c, int32_t blk0) {
-  return SplitK{c.step2.p, c.blk2.p, c.base.p, c.crow.p, c.hnum.p, c.rec.p, blk0};
+  return SplitK{c.step2.p, c.blk2.p, c.base.p, c.hnum.p, c.rec.p, blk0};
 }
 
 }  // namespace xcal

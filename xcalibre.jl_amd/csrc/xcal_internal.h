@@ -290,8 +290,8 @@ struct xcal_mesh {
     xcal::DBuf<uint16_t> lidx;
     std::vector<int32_t> band;  // host: first block of each band (nbands + 1)
     // the same steps with rows packed for the split CG (sweep_split.h): steps
-    // padded per block, one record per position, nz slots of the entry pairs
-    // (pair 0 is empty)
+    // padded per block, one record per position (rows in that CG's order), nz
+    // slots of the entry pairs (pair 0 is empty)
     xcal::DBuf<int32_t> step2, blk2, pslot;
     xcal::DBuf<int4> rec;
     int nblk() const { return band.empty() ? 0 : band.back(); }
@@ -300,6 +300,7 @@ struct xcal_mesh {
   xcal::DBuf<int32_t> cone_own, cone_ownp;
   bool cone = false;
   int cone_nblk = 0, cone_rows = 0;  // forward blocks, rows per block
+  xcal::DBuf<int32_t> split_rows;  // device row of each position of the split CG's row order
   bool split = false;  // the split CG's tables were built (rows of at most 6 entries per triangle)
   bool cone_deep = false;            // deep prefetch (XCAL_CONE_DEEP=1 at creation)
   Cone cone_f, cone_b;
