@@ -832,7 +832,7 @@ static bool bread(BSolver<T>& S) {
   prof_resolve(S.m->ctx);
   const KS* h = (const KS*)S.e->kstate_host;
   for (int k = 0; k < S.ncase; ++k)
-    if (h[k].stop == STOP_NONE) return false;
+    if (!resident_done(h[k].stop, h[k].gave_up)) return false;
   return true;
 }
 
@@ -1023,7 +1023,7 @@ static void bcg(BSolver<T>& S, int precon, const T* b, T* x0, int itmax, double 
     F.flush();
     PersistLease lease;
     resident = persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease);
-    if (resident && !bread(S)) {  // its waits were given up: start over by launches
+    if (resident && !bread(S)) {  // waits given up: start over by launches
       persist_failed(S.m);
       bcg(S, precon, b, x0, itmax, atol, rtol, frozen, xsol);
       return;

@@ -25,9 +25,12 @@
 //
 // All workgroups must be resident at once.  The host launches at most one
 // workgroup per compute unit over all solves in flight in the process
-// (persist_acquire), and every wait is bounded in time: past the bound a
-// workgroup raises the abort word, all return without writing the state, and
-// the host, finding the state still running, solves by launches instead.
+// (PersistLease::acquire), and every wait is bounded in time: past the bound a
+// workgroup raises the abort word, marks its case's state and returns without
+// its rows of x, and so does each one that then waits in vain.  At the last
+// meeting the others may still find every sum and finish, so the host takes a
+// case's result only where the state has stopped and is not marked
+// (resident_done); otherwise it solves by launches from the start.
 //
 // Measured per CG iteration on one MI355X, launch chain then resident (2D
 // k-omega steps, Jacobi): 8.8k rows 11.9 to 5.5 us, 130.7k rows 17.2 to 5.2
@@ -144,17 +147,20 @@ __device__ inline bool persist_read(const PersistK& P, int nwg, const unsigned l
       const int i = at(v);
       long long t0 = 0;
       for (int spin = 0; u[v] == kUnset; ++spin) {
-        // bounded: give up past the limit or when another did
+        // bounded: give up past the limit or when another did, but not on a
+        // word that was set while this wavefront was held up
+        bool late = false;
         if ((spin & 63) == 63 || P.limit <= 0) {
           const long long now = wall_clock64();
           if (t0 == 0) t0 = now;
-          if (now - t0 >= P.limit) dev_store(P.abort, 1);
-          if (dev_load(P.abort) != 0) {
-            L.fail = 1;
-            break;
-          }
+          late = now - t0 >= P.limit || dev_load(P.abort) != 0;
         }
         u[v] = dev_load(area + i);
+        if (late && u[v] == kUnset) {
+          dev_store(P.abort, 1);
+          L.fail = 1;
+          break;
+        }
       }
       L.word[i] = __longlong_as_double((long long)u[v]);
     }
@@ -198,6 +204,11 @@ __device__ inline double persist_total(const PersistK& P, const PersistSlots& R,
   if (t == 0)
     for (int w = 0; w < kBlock / 64; ++w) a += L.lds[w];
   return a;
+}
+
+// A workgroup that leaves before the end of its case's solve marks the state.
+__device__ inline void persist_leave(KS* ks) {
+  if (threadIdx.x == 0) dev_store(&ks->gave_up, 1);
 }
 
 // The resident solve of one case by its workgroups.  LOCAL: the case has one
@@ -277,7 +288,7 @@ __device__ inline void cg_persist_case(const PersistK& P, const int4 wg, const M
     }
     unsigned long long *lA = aA + par * P.words, *lB = aB + par * P.words;
     persist_publish<LOCAL, false>(s, lA + line, L);
-    if (!LOCAL && !persist_read<KR>(P, cwg.y, lA, L)) return;
+    if (!LOCAL && !persist_read<KR>(P, cwg.y, lA, L)) return persist_leave(ks + wg.z);
     double tot = persist_total<LOCAL, KR>(P, RA, L);
     if (threadIdx.x == 0) {
       finalize(&k, FIN_CG_PAP, tot, 0.0);
@@ -310,7 +321,7 @@ __device__ inline void cg_persist_case(const PersistK& P, const int4 wg, const M
       dev_store(aB + (par ^ 1) * P.words + line + threadIdx.x, kUnset);
     }
     persist_publish<LOCAL, true>(s, lB + line, L);
-    if (!LOCAL && !persist_read<KR>(P, cwg.y, lB, L)) return;
+    if (!LOCAL && !persist_read<KR>(P, cwg.y, lB, L)) return persist_leave(ks + wg.z);
     gather();  // every new z is there: its loads overlap the sum
     tot = persist_total<LOCAL, KR>(P, RB, L);
     if (threadIdx.x == 0) {

@@ -143,9 +143,9 @@ static __global__ void __launch_bounds__(kBlock)
 // Launches the CG iterations of every case from the state `ks` and the start
 // vectors r and z = S r, to each case's stop; x receives the corrections of
 // the cases that ran.  False, with nothing launched, where the mesh has no
-// plan or the device no room.  The caller reads the states: a case still
-// running (STOP_NONE) means the waits were given up, and persist_failed()
-// keeps the mesh on the launch chain from then on.
+// plan or the device no room.  The caller reads the states: where a case is
+// not resident_done(), waits were given up, and persist_failed() keeps the
+// mesh on the launch chain from then on.
 template <class T>
 bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T* z, KS* ks,
                 PersistLease& lease) {

@@ -1224,7 +1224,7 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
     PersistLease lease;
     if (persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease)) {
       st = read_state(S);
-      if (st.stop == STOP_NONE) {  // its waits were given up: start over by launches
+      if (!resident_done(st.stop, st.gave_up)) {  // waits given up: start over by launches
         persist_failed(S.m);
         return cg(S, precon, b, x0, itmax, atol, rtol, niter, xsol);
       }

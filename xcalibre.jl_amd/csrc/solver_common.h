@@ -3,6 +3,7 @@
 #pragma once
 
 #include "device_common.h"
+#include "resident.h"
 
 namespace xcal {
 
@@ -14,7 +15,8 @@ enum : int { STOP_NONE = 0, STOP_SOLVED = 1, STOP_ITMAX = 2, STOP_BREAKDOWN = 3,
 
 struct KS {
   double gamma, pAp, alpha, beta, rNorm, eps, pNorm2, rho, next_rho, omega, atol, rtol;
-  int iter, itmax, stop, err;
+  int iter, itmax, stop;
+  int gave_up;  // a workgroup of a resident solve left early (resident.h)
 };
 static_assert(sizeof(KS) <= 32 * sizeof(double), "the context's zeroed state holds one KS");
 
