@@ -26,3 +26,28 @@ def test_field_round_trip_in_reference_numbering(x, shape):
     g = H.Field(dm, A.FACE_SCALAR).fill(1.0)
     eq.discretise([(A.LAPLACIAN_LINEAR, -1, g)], [(H.Field(dm, A.CELL_SCALAR).upload(src), 1)])
     assert np.array_equal(eq.download()[1], src * np.asarray(mesh.cell_volume))
+
+
+def test_transfers_of_one_mesh_from_several_threads(x):
+    """Uploads and downloads of different fields of one mesh at the same time,
+    of lengths that make the transfer buffer grow in between: every thread gets
+    its own values back."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    A, H = x._abi, x.hip
+    ctx = x.api._context(0)
+    mesh = x.mesh.box3d(41, 40, 43, jitter=0.1)
+    dm = H.DeviceMesh(ctx, mesh)
+    kinds = (A.CELL_SCALAR, A.FACE_SCALAR, A.CELL_VECTOR, A.FACE_VECTOR)
+    fields = [H.Field(dm, k) for k in kinds]
+
+    def work(i):
+        f, rng = fields[i], np.random.default_rng(i)
+        for _ in range(12):
+            v = rng.standard_normal((f.ncomp, f.len))
+            if not np.array_equal(f.upload(v).download().reshape(v.shape), v):
+                return False
+        return True
+
+    with ThreadPoolExecutor(len(kinds)) as ex:
+        assert all(ex.map(work, range(len(kinds))))

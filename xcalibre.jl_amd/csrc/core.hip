@@ -1818,7 +1818,9 @@ static __global__ void __launch_bounds__(kBlock)
   if (i < n) dev[perm[i]] = in[i];
 }
 
-// The mesh's transfer buffer, at least len values.
+// The mesh's transfer buffer, at least len values.  Transfers of one mesh's
+// fields may be called from several threads; each holds stage_mu until the
+// stream has been waited for.
 static double* stage(const xcal_mesh* m, int64_t len) {
   if (m->stage.n < len) {
     XCAL_HIP(hipStreamSynchronize(m->ctx->stream));  // a replaced buffer may be in use
@@ -1829,6 +1831,7 @@ static double* stage(const xcal_mesh* m, int64_t len) {
 void upload_permuted(const xcal_mesh* m, const int32_t* perm, double* dev, const double* host,
                      int64_t len) {
   if (len <= 0) return;
+  std::lock_guard<std::mutex> hold(m->stage_mu);
   hipStream_t s = m->ctx->stream;
   double* t = stage(m, len);
   XCAL_HIP(hipMemcpyAsync(t, host, sizeof(double) * len, hipMemcpyHostToDevice, s));
@@ -1840,6 +1843,7 @@ void upload_permuted(const xcal_mesh* m, const int32_t* perm, double* dev, const
 void download_permuted(const xcal_mesh* m, const int32_t* perm, const double* dev, double* host,
                        int64_t len) {
   if (len <= 0) return;
+  std::lock_guard<std::mutex> hold(m->stage_mu);
   hipStream_t s = m->ctx->stream;
   double* t = stage(m, len);
   hipLaunchKernelGGL(k_gather_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm, dev, t);

@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <stdexcept>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <map>
 #include <array>
@@ -213,7 +214,9 @@ struct xcal_mesh {
   // nzperm maps reference CSR slots to device slots
   std::vector<int32_t> cperm, fperm, nzperm;
   xcal::DBuf<int32_t> cperm_d, fperm_d;  // the same on the device, for field transfers
-  mutable xcal::DBuf<double> stage;      // their buffer, of the largest field moved so far
+  // their buffer, of the largest field moved so far, held by one transfer at a time
+  mutable xcal::DBuf<double> stage;
+  mutable std::mutex stage_mu;
   // CSR pattern in the reference's numbering (host only)
   std::vector<int32_t> h_rowptr, h_colval;
   // device matrix storage (sliced ELL): entries of row c at
