@@ -1,20 +1,23 @@
-"""Fields cross the C ABI renumbered on the device: what goes up comes back
-bit for bit, per component and in the reference numbering (an equation built
-from an uploaded source keeps each value in its cell's row)."""
+"""Fields cross the C ABI renumbered, by host loops or on the device: what goes
+up comes back bit for bit, per component and in the reference numbering (an
+equation built from an uploaded source keeps each value in its cell's row)."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 8, 8), (3, 5, 17), (16, 16, 17)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 8, 8), (3, 5, 17), (16, 16, 17),
+                                   (48, 32, 32), (49153, 1, 1)])
 def test_field_round_trip_in_reference_numbering(x, shape):
     A, H = x._abi, x.hip
     ctx = x.api._context(0)
     mesh = x.mesh.box3d(*shape, jitter=0.1)
     dm = H.DeviceMesh(ctx, mesh)
     rng = np.random.default_rng(1)
-    # face fields last: the transfer buffer grows between the calls
+    # face fields last: the transfer buffer grows between the calls.  Cell or
+    # face counts on both sides of 49 152, where kernels take over from host
+    # loops, and just at it
     for kind in (A.CELL_SCALAR, A.CELL_VECTOR, A.CELL_TENSOR, A.FACE_SCALAR, A.FACE_VECTOR):
         f = H.Field(dm, kind)
         v = rng.standard_normal((f.ncomp, f.len))

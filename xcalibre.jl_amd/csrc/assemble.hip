@@ -364,7 +364,7 @@ int xcal_eqn_download(const xcal_eqn* e, int32_t which, int32_t comp, double* nz
       XCAL_HIP(hipStreamSynchronize(m->ctx->stream));
       for (int64_t k = 0; k < m->nnz; ++k) nzval[k] = t[m->nzperm[k]];
     }
-    if (b) download_permuted(m, m->cperm_d.p, e->bc(comp), b, m->n);
+    if (b) download_permuted(m, {m->cperm.data(), m->cperm_d.p}, e->bc(comp), b, m->n);
     return 0;
   });
 }

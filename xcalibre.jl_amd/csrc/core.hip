@@ -1796,15 +1796,22 @@ int xcal_field_destroy(xcal_field* f) {
 
 namespace xcal {
 // reference id -> device id map of a field's entities
-static const int32_t* field_perm(const xcal_field* f) {
-  return (f->kind == XCAL_FACE_SCALAR || f->kind == XCAL_FACE_VECTOR) ? f->mesh->fperm_d.p
-                                                                      : f->mesh->cperm_d.p;
+static Renumber field_perm(const xcal_field* f) {
+  const xcal_mesh* m = f->mesh;
+  if (f->kind == XCAL_FACE_SCALAR || f->kind == XCAL_FACE_VECTOR)
+    return {m->fperm.data(), m->fperm_d.p};
+  return {m->cperm.data(), m->cperm_d.p};
 }
 
-// Renumbering of a field that crosses the C ABI: out[i] = dev[perm[i]] and
-// dev[perm[i]] = in[i].  The host loops these replace took 8.7 ms per
-// 32 MB component of a 4.0M-cell batch down and 6.1 ms up, most of it cache
-// misses and the page faults of a scratch copy.
+// Up to this many values a host loop renumbers a field that crosses the C ABI,
+// above it a kernel: out[i] = dev[perm[i]] and dev[perm[i]] = in[i].  Upload
+// and download in microseconds, loop then kernel (one MI355X): 5.8k values 14
+// and 14, 23 and 26; 19.7k 22 and 23, 28 and 31; 38k natural 32 and 33, 36
+// and 37; 45k natural 36 and 37, 41 and 39; 53k natural 44 and 46, 40 and 42;
+// 69k 59 and 57, 42 and 49; a 32 MB component of a 4.0M-cell batch took the
+// loop 6.1 ms up and 8.7 ms down, most of it cache misses and the page faults
+// of a scratch copy.
+constexpr int64_t kHostRenumber = 49152;
 static __global__ void __launch_bounds__(kBlock)
     k_gather_perm(int64_t n, const int32_t* __restrict__ perm, const double* __restrict__ dev,
                   double* __restrict__ out) {
@@ -1828,25 +1835,41 @@ static double* stage(const xcal_mesh* m, int64_t len) {
   }
   return m->stage.p;
 }
-void upload_permuted(const xcal_mesh* m, const int32_t* perm, double* dev, const double* host,
+void upload_permuted(const xcal_mesh* m, const Renumber& perm, double* dev, const double* host,
                      int64_t len) {
   if (len <= 0) return;
-  std::lock_guard<std::mutex> hold(m->stage_mu);
   hipStream_t s = m->ctx->stream;
+  if (len <= kHostRenumber) {
+    std::vector<double> t(len);
+    for (int64_t i = 0; i < len; ++i) t[perm.host[i] - perm.base] = host[i];
+    XCAL_HIP(hipMemcpyAsync(dev + perm.base, t.data(), sizeof(double) * len, hipMemcpyHostToDevice,
+                            s));
+    XCAL_HIP(hipStreamSynchronize(s));
+    return;
+  }
+  std::lock_guard<std::mutex> hold(m->stage_mu);
   double* t = stage(m, len);
   XCAL_HIP(hipMemcpyAsync(t, host, sizeof(double) * len, hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_scatter_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm,
+  hipLaunchKernelGGL(k_scatter_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm.dev,
                      (const double*)t, dev);
   XCAL_HIP(hipGetLastError());
   XCAL_HIP(hipStreamSynchronize(s));
 }
-void download_permuted(const xcal_mesh* m, const int32_t* perm, const double* dev, double* host,
+void download_permuted(const xcal_mesh* m, const Renumber& perm, const double* dev, double* host,
                        int64_t len) {
   if (len <= 0) return;
-  std::lock_guard<std::mutex> hold(m->stage_mu);
   hipStream_t s = m->ctx->stream;
+  if (len <= kHostRenumber) {
+    std::vector<double> t(len);
+    XCAL_HIP(hipMemcpyAsync(t.data(), dev + perm.base, sizeof(double) * len, hipMemcpyDeviceToHost,
+                            s));
+    XCAL_HIP(hipStreamSynchronize(s));
+    for (int64_t i = 0; i < len; ++i) host[i] = t[perm.host[i] - perm.base];
+    return;
+  }
+  std::lock_guard<std::mutex> hold(m->stage_mu);
   double* t = stage(m, len);
-  hipLaunchKernelGGL(k_gather_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm, dev, t);
+  hipLaunchKernelGGL(k_gather_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm.dev, dev, t);
   XCAL_HIP(hipGetLastError());
   XCAL_HIP(hipMemcpyAsync(host, t, sizeof(double) * len, hipMemcpyDeviceToHost, s));
   XCAL_HIP(hipStreamSynchronize(s));

@@ -650,7 +650,8 @@ void simple_case_field(const xcal_simple* S, int which, int k, double* host) {
   XCAL_CHECK(f, "unknown cell field selector (or no turbulence model)");
   const int64_t c0 = m->case_cell[k], nk = m->case_cell[k + 1] - c0;
   for (int c = 0; c < f->ncomp; ++c)
-    download_permuted(m, m->cperm_d.p + c0, f->comp(c), host + (int64_t)c * nk, nk);
+    download_permuted(m, {m->cperm.data() + c0, m->cperm_d.p + c0, c0}, f->comp(c),
+                      host + (int64_t)c * nk, nk);
 }
 
 }  // namespace xcal

@@ -479,11 +479,17 @@ void simple_case_field(const xcal_simple* S, int which, int k, double* host);
 // the k-omega fields
 int64_t prepared_footprint(const PreparedMesh& P, bool turb = false);
 int64_t prepared_cells(const PreparedMesh& P);
-// dev[perm[i]] = host[i] and host[i] = dev[perm[i]], i < len, renumbered on
-// the device (perm is a device array: cperm_d, fperm_d or a part of one)
-void upload_permuted(const xcal_mesh* m, const int32_t* perm, double* dev, const double* host,
+// Renumbering of values that cross the C ABI: reference id -> device id, on
+// the host and on the device, for ids that fill [base, base + length).
+struct Renumber {
+  const int32_t* host;
+  const int32_t* dev;
+  int64_t base = 0;
+};
+// dev[perm[i]] = host[i] and host[i] = dev[perm[i]], i < len
+void upload_permuted(const xcal_mesh* m, const Renumber& perm, double* dev, const double* host,
                      int64_t len);
-void download_permuted(const xcal_mesh* m, const int32_t* perm, const double* dev, double* host,
+void download_permuted(const xcal_mesh* m, const Renumber& perm, const double* dev, double* host,
                        int64_t len);
 TermsK make_terms(const xcal_term* terms, int n);
 BCsK make_bcs(const xcal_mesh* m, const xcal_bc* bcs, int n);
