@@ -54,3 +54,20 @@ def test_transfers_of_one_mesh_from_several_threads(x):
 
     with ThreadPoolExecutor(len(kinds)) as ex:
         assert all(ex.map(work, range(len(kinds))))
+
+
+def test_transfer_while_another_device_is_current(x):
+    """A field on device 0 moves through a buffer of device 0 while a later
+    context has made device 1 the thread's current one."""
+    import torch
+
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    A, H = x._abi, x.hip
+    mesh = x.mesh.box3d(41, 40, 43, jitter=0.1)
+    dm = H.DeviceMesh(H.Context(0), mesh)
+    f = H.Field(dm, A.CELL_SCALAR)
+    other = H.Context(1)
+    v = np.random.default_rng(4).standard_normal(f.len)
+    assert np.array_equal(f.upload(v).download(), v)
+    del other

@@ -1825,6 +1825,22 @@ static __global__ void __launch_bounds__(kBlock)
   if (i < n) dev[perm[i]] = in[i];
 }
 
+// The thread's device is `device` while this lives (a launch and an allocation
+// need it; a copy on a stream does not).
+struct OnDevice {
+  int prev = 0;
+  explicit OnDevice(int device) {
+    XCAL_HIP(hipGetDevice(&prev));
+    if (prev == device) prev = -1;
+    else XCAL_HIP(hipSetDevice(device));
+  }
+  ~OnDevice() {
+    if (prev >= 0) (void)hipSetDevice(prev);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+};
+
 // The mesh's transfer buffer, at least len values.  Transfers of one mesh's
 // fields may be called from several threads; each holds stage_mu until the
 // stream has been waited for.
@@ -1848,6 +1864,7 @@ void upload_permuted(const xcal_mesh* m, const Renumber& perm, double* dev, cons
     return;
   }
   std::lock_guard<std::mutex> hold(m->stage_mu);
+  OnDevice on(m->ctx->device);
   double* t = stage(m, len);
   XCAL_HIP(hipMemcpyAsync(t, host, sizeof(double) * len, hipMemcpyHostToDevice, s));
   hipLaunchKernelGGL(k_scatter_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm.dev,
@@ -1868,6 +1885,7 @@ void download_permuted(const xcal_mesh* m, const Renumber& perm, const double* d
     return;
   }
   std::lock_guard<std::mutex> hold(m->stage_mu);
+  OnDevice on(m->ctx->device);
   double* t = stage(m, len);
   hipLaunchKernelGGL(k_gather_perm, dim3(grid_for(len)), dim3(kBlock), 0, s, len, perm.dev, dev, t);
   XCAL_HIP(hipGetLastError());
