@@ -223,6 +223,18 @@ int xcal_mesh_cone_form(const xcal_mesh* mesh, int32_t* block_rows, int32_t* blo
 /* Bands (launches) per sweep of the cone form: forward, backward (0: level
  * launches).  No reference counterpart. */
 int xcal_mesh_cone_bands(const xcal_mesh* mesh, int32_t* fwd_bands, int32_t* bwd_bands);
+/* Lean one-workgroup DILU sweeps: rows their LDS rings hold (4096 or 8192),
+ * forward and backward; 0 where the sweeps take another form.  No reference
+ * counterpart (reports a device code path). */
+int xcal_mesh_lean_form(const xcal_mesh* mesh, int32_t* fwd_ring, int32_t* bwd_ring);
+/* CG with a diagonal (or no) preconditioner as one resident launch: its
+ * workgroups (0 before the mesh's first such solve, and where it does not
+ * fit), the solves started so, those of them whose waits were given up (the
+ * mesh's solves are launch chains from then on), and the solves that found no
+ * room on the device.  Results do not depend on the form.  No reference
+ * counterpart. */
+int xcal_mesh_resident(const xcal_mesh* mesh, int32_t* workgroups, int64_t* solves,
+                       int64_t* given_up, int64_t* refused);
 /* CSR pattern, 0-based (rowptr n+1, colval nnz) */
 int xcal_mesh_csr_pattern(const xcal_mesh* mesh, int32_t* rowptr, int32_t* colval);
 

@@ -71,6 +71,8 @@ def test_lean_sweeps_equal_level_stepping(x, A, ctx, monkeypatch, shape):
             monkeypatch.setenv("XCAL_NO_PIPE", "1")
         dm = H.DeviceMesh(ctx, mesh)
         monkeypatch.delenv("XCAL_NO_PIPE", raising=False)
+        assert dm.lean_form() == ((0, 0) if off else (8192, 8192) if shape == ("step", 104)
+                                  else (4096, 4096))  # the ring
         got = []
         for solver, prec in (("SOLVER_CG", "PREC_FP64"), ("SOLVER_BICGSTAB", "PREC_FP64"),
                              ("SOLVER_CG", "PREC_FP32_IR"), ("SOLVER_BICGSTAB", "PREC_FP32_IR")):
@@ -89,12 +91,14 @@ def test_lean_sweeps_equal_level_stepping(x, A, ctx, monkeypatch, shape):
 def test_lean_batch_sweeps_equal_level_stepping(x, A, ctx, monkeypatch, shapes):
     H = x.hip
     ms = [_mesh(x, s) for s in shapes]
+    monkeypatch.setenv("XCAL_PIPE_ROWS", "1")  # the lean body's rows per thread
     out = []
     for off in (False, True):
         if off:
             monkeypatch.setenv("XCAL_NO_PIPE", "1")
         dm = H.DeviceMesh.batch(ctx, ms)
         monkeypatch.delenv("XCAL_NO_PIPE", raising=False)
+        assert dm.lean_form() == ((0, 0) if off else (4096, 4096))
         got = []
         for solver, prec in (("SOLVER_CG", "PREC_FP64"), ("SOLVER_BICGSTAB", "PREC_FP64"),
                              ("SOLVER_CG", "PREC_FP32_IR")):

@@ -5,7 +5,8 @@ The resident solve adds the same row sums and partial sums in the same order
 as the chain (XCAL_NO_PERSIST=1 at mesh creation), so fields, residuals and
 iteration counts are equal.  Sizes sit at the edges of its tiles: 64-row
 groups, one workgroup of 512 rows (no meeting between workgroups), a second
-one, two rows per thread, and more rows than it takes."""
+one, two rows per thread, the most it takes (256 workgroups, 262 144 rows), and
+more.  The mesh's counts say which form ran."""
 import numpy as np
 import pytest
 
@@ -25,7 +26,8 @@ def _mesh(x, shape):
 
 
 def _solve(x, mesh, prec, monkeypatch, **env):
-    """One pressure-like CG solve (Jacobi, singular-free by a fixed patch)."""
+    """Two pressure-like CG solves (Jacobi, singular-free by a fixed patch) and
+    the mesh's resident counts."""
     A, H = x._abi, x.hip
     ctx = x.api._context(0)
     for k, v in env.items():
@@ -50,56 +52,90 @@ def _solve(x, mesh, prec, monkeypatch, **env):
         eq.precond_update(A.PRECON_JACOBI)
         n, res, rc = eq.solve(setup, phi)
         out.append((n, res, rc, phi.download()))
-    return out
+    return out, dm.resident()
 
 
 def _same(a, b):
-    assert len(a) == len(b)
-    for u, v in zip(a, b):
+    """Equal solves; the second side ran by launches alone."""
+    assert len(a[0]) == len(b[0])
+    assert b[1] == (0, 0, 0, 0)
+    for u, v in zip(a[0], b[0]):
         assert u[:3] == v[:3]
         assert np.array_equal(u[3], v[3])
 
 
 @pytest.mark.parametrize("shape", [(1, 1), (5, 1), (8, 8), (13, 5), (32, 16), (27, 19), (64, 16),
-                                   (131, 67), (300, 117), (511, 129), (11, 13, 9), (600, 450)])
+                                   (131, 67), (300, 117), (511, 129), (11, 13, 9), (512, 511),
+                                   (512, 512), (513, 512), (600, 450)])
 @pytest.mark.parametrize("prec", ["fp64", "fp32-ir"])
 def test_resident_cg_equals_launch_chain(x, monkeypatch, shape, prec):
     mesh = _mesh(x, shape)
     p = {"fp64": x._abi.PREC_FP64, "fp32-ir": x._abi.PREC_FP32_IR}[prec]
-    _same(_solve(x, mesh, p, monkeypatch),
-          _solve(x, mesh, p, monkeypatch, XCAL_NO_PERSIST="1"))
+    a = _solve(x, mesh, p, monkeypatch)
+    _same(a, _solve(x, mesh, p, monkeypatch, XCAL_NO_PERSIST="1"))
+    wgs, solves, given_up, refused = a[1]
+    n, k = mesh.n_cells, 1 if mesh.n_cells <= 64 * 512 else 2  # rows per thread
+    if n <= 1 << 18:
+        assert wgs == -(-n // (512 * k)) and solves >= 2 and given_up == refused == 0
+    else:
+        assert a[1] == (0, 0, 0, 0)
 
 
 @pytest.mark.parametrize("shape", [(27, 19), (131, 67)])
 def test_resident_cg_gives_up_to_launch_chain(x, monkeypatch, shape):
-    """With no time to wait, the resident solve may give up; the solve then
-    runs by launches and the result is the same."""
+    """With no time to wait, the first resident solve gives up (some workgroup
+    of some meeting comes first); this solve and those after it run by launches
+    and the results are the same."""
     mesh = _mesh(x, shape)
-    _same(_solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_PERSIST_WAIT_US="0"),
-          _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_NO_PERSIST="1"))
+    a = _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_PERSIST_WAIT_US="0")
+    _same(a, _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_NO_PERSIST="1"))
+    assert a[1][1:] == (1, 1, 0)
 
 
-@pytest.mark.parametrize("sizes", [(5,), (12, 40, 16, 23), (90, 33, 64, 8, 150)])
-@pytest.mark.parametrize("prec", ["fp64", "fp32-ir"])
-def test_resident_batch_cg_equals_launch_chain(x, monkeypatch, sizes, prec):
+def _batch(x, sizes, prec, monkeypatch, **env):
     api, H = x.api, x.hip
     ctx = api._context(0)
     ms = [x.mesh.cavity2d(n) for n in sizes]
     model, config = cavity_case(api, ms[0], iterations=8, precon="Jacobi", rtol_p=1e-3,
                                 precision_p=prec)
     setup = api.simple_setup(model, config, pref=0.0)
-    runs = []
-    for off in (False, True):
-        if off:
-            monkeypatch.setenv("XCAL_NO_PERSIST", "1")
-        dm = H.DeviceMesh.batch(ctx, ms)
-        monkeypatch.delenv("XCAL_NO_PERSIST", raising=False)
-        sim = H.Simple(dm, setup)
-        sim.set_case_nu(np.linspace(0.0025, 0.01, len(ms)))
-        out = sim.run_batch(8)
-        runs.append((out, sim.get("U"), sim.get("p")))
-    (a, Ua, pa), (b, Ub, pb) = runs
-    assert a["done"] == b["done"] == 8
-    assert np.array_equal(a["krylov_iters"], b["krylov_iters"])
-    assert np.array_equal(a["residuals"], b["residuals"])
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    dm = H.DeviceMesh.batch(ctx, ms)
+    for k in env:
+        monkeypatch.delenv(k)
+    sim = H.Simple(dm, setup)
+    sim.set_case_nu(np.linspace(0.0025, 0.01, len(ms)))
+    out = sim.run_batch(8)
+    return out, sim.get("U"), sim.get("p"), dm.resident()
+
+
+def _same_batch(a, b):
+    (oa, Ua, pa, _), (ob, Ub, pb, counts) = a, b
+    assert counts == (0, 0, 0, 0)
+    assert oa["done"] == ob["done"] == 8
+    assert np.array_equal(oa["krylov_iters"], ob["krylov_iters"])
+    assert np.array_equal(oa["residuals"], ob["residuals"])
     assert np.array_equal(Ua, Ub) and np.array_equal(pa, pb)
+
+
+# the last two: 256 workgroups of one case each, and one case more than fits
+@pytest.mark.parametrize("sizes", [(5,), (12, 40, 16, 23), (90, 33, 64, 8, 150), (4,) * 256,
+                                   (4,) * 257])
+@pytest.mark.parametrize("prec", ["fp64", "fp32-ir"])
+def test_resident_batch_cg_equals_launch_chain(x, monkeypatch, sizes, prec):
+    a = _batch(x, sizes, prec, monkeypatch)
+    _same_batch(a, _batch(x, sizes, prec, monkeypatch, XCAL_NO_PERSIST="1"))
+    wgs, solves, given_up, refused = a[3]
+    if len(sizes) <= 256:
+        assert len(sizes) <= wgs <= 256 and solves >= 8 and given_up == refused == 0
+    else:
+        assert a[3] == (0, 0, 0, 0)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32-ir"])
+def test_resident_batch_cg_gives_up_to_launch_chain(x, monkeypatch, prec):
+    sizes = (90, 33, 64, 8, 150)
+    a = _batch(x, sizes, prec, monkeypatch, XCAL_PERSIST_WAIT_US="0")
+    _same_batch(a, _batch(x, sizes, prec, monkeypatch, XCAL_NO_PERSIST="1"))
+    assert a[3][1:] == (1, 1, 0)

@@ -1750,6 +1750,27 @@ int xcal_mesh_sweep_form(const xcal_mesh* m, int32_t* fwd, int32_t* bwd) {
   });
 }
 
+int xcal_mesh_lean_form(const xcal_mesh* m, int32_t* fwd, int32_t* bwd) {
+  return guarded([&] {
+    XCAL_CHECK(m && fwd && bwd, "NULL argument");
+    *fwd = m->lean ? m->lean_f.ring : 0;
+    *bwd = m->lean ? m->lean_b.ring : 0;
+    return 0;
+  });
+}
+
+int xcal_mesh_resident(const xcal_mesh* m, int32_t* workgroups, int64_t* solves, int64_t* given_up,
+                       int64_t* refused) {
+  return guarded([&] {
+    XCAL_CHECK(m && workgroups && solves && given_up && refused, "NULL argument");
+    *workgroups = persist_workgroups(m);
+    *solves = m->persist_runs;
+    *given_up = m->persist_left;
+    *refused = m->persist_full;
+    return 0;
+  });
+}
+
 int xcal_mesh_csr_pattern(const xcal_mesh* m, int32_t* rowptr, int32_t* colval) {
   return guarded([&] {
     XCAL_CHECK(m && rowptr && colval, "NULL argument");

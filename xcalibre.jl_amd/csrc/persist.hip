@@ -153,7 +153,11 @@ bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T*
   if (!m->persist_on || m->ctx->prof_on[0]) return false;
   if (!m->persist) m->persist = make_plan(m);
   const PersistPlan& P = *m->persist;
-  if (!P.ok || !lease.acquire(m->ctx->device, P.nwg, compute_units(m->ctx->device))) return false;
+  if (!P.ok) return false;
+  if (!lease.acquire(m->ctx->device, P.nwg, compute_units(m->ctx->device))) {
+    m->persist_full++;
+    return false;
+  }
   if (e->parea.n < 4 * P.words + 1) e->parea.alloc(4 * P.words + 1);
   PersistK K;
   K.wg = P.wg.p;
@@ -179,6 +183,7 @@ bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T*
     else go(k_cg_persist<G, 2, T>);
   });
   XCAL_HIP(hipGetLastError());
+  m->persist_runs++;
   return true;
 }
 template bool persist_cg<double>(xcal_eqn*, const MatKT<double>&, const double*, double*,
@@ -186,7 +191,13 @@ template bool persist_cg<double>(xcal_eqn*, const MatKT<double>&, const double*,
 template bool persist_cg<float>(xcal_eqn*, const MatKT<float>&, const float*, float*, const float*,
                                 float*, KS*, PersistLease&);
 
-void persist_failed(const xcal_mesh* m) { m->persist_on = false; }
+void persist_failed(const xcal_mesh* m) {
+  m->persist_on = false;
+  m->persist_left++;
+}
+int persist_workgroups(const xcal_mesh* m) {
+  return m->persist && m->persist->ok ? m->persist->nwg : 0;
+}
 
 // Knobs, read when the mesh is created: XCAL_NO_PERSIST=1 keeps the launch
 // chain (as XCAL_NO_FUSE=1 does), XCAL_PERSIST_WAIT_US bounds each wait.

@@ -229,6 +229,8 @@ struct xcal_mesh {
   mutable bool persist_on = true;
   long long persist_ticks = 100000000;
   mutable std::shared_ptr<xcal::PersistPlan> persist;
+  // resident launches, those given up, and solves that found no room
+  mutable int64_t persist_runs = 0, persist_left = 0, persist_full = 0;
   xcal::DBuf<int32_t> rbeg, rend, colval, trans;
   xcal::DBuf<int32_t> sinfo;  // per slice of kSlice rows: first slot, width (entries)
   // DILU level schedules: forward level l = device rows
@@ -432,6 +434,7 @@ struct BCsK {
 
 void make_sweep_plans(xcal_mesh* m, int small);
 void persist_configure(xcal_mesh* m);
+int persist_workgroups(const xcal_mesh* m);  // of the plan, 0 where there is none
 // meshes built on the host first (server admission), uploaded later
 struct PreparedMesh;
 // Host build of one mesh or a batch.  With `ingest`, the CSR pattern, slot

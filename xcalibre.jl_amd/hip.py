@@ -55,6 +55,8 @@ def lib():
             "xcal_mesh_pipe_tuning": [_vp, _pi32, _pi32, _pd],
             "xcal_mesh_cone_form": [_vp, _pi32, _pi32, C.POINTER(C.c_int64), C.POINTER(C.c_int64)],
             "xcal_mesh_cone_bands": [_vp, _pi32, _pi32],
+            "xcal_mesh_lean_form": [_vp, _pi32, _pi32],
+            "xcal_mesh_resident": [_vp, _pi32] + [C.POINTER(C.c_int64)] * 3,
             "xcal_solve_system_batch": [_vp, C.POINTER(A.SolverSetupC), _vp, C.c_int32,
                                         C.POINTER(A.SolveStats)],
             "xcal_simple_run_batch": [_vp, C.c_int32, _pd, _pi32, _pi32],
@@ -276,6 +278,19 @@ class DeviceMesh:
         f, b = C.c_int64(), C.c_int64()
         check(lib().xcal_mesh_cone_form(self.h, C.byref(r), C.byref(nb), C.byref(f), C.byref(b)))
         return r.value, nb.value, f.value, b.value
+
+    def lean_form(self):
+        """(forward, backward) LDS ring rows of the lean one-workgroup sweeps;
+        (0, 0) where the sweeps take another form."""
+        f, b = C.c_int32(), C.c_int32()
+        check(lib().xcal_mesh_lean_form(self.h, C.byref(f), C.byref(b)))
+        return f.value, b.value
+
+    def resident(self):
+        """(workgroups, solves started, given up, refused) of the resident CG."""
+        w, v = C.c_int32(), [C.c_int64() for _ in range(3)]
+        check(lib().xcal_mesh_resident(self.h, C.byref(w), *map(C.byref, v)))
+        return (w.value, *(c.value for c in v))
 
     def csr_pattern(self):
         rp = np.zeros(self.n + 1, np.int32)
