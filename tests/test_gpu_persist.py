@@ -7,6 +7,10 @@ iteration counts are equal.  Sizes sit at the edges of its tiles: 64-row
 groups, one workgroup of 512 rows (no meeting between workgroups), a second
 one, two rows per thread, the most it takes (256 workgroups, 262 144 rows), and
 more.  The mesh's counts say which form ran."""
+import fcntl
+import glob
+import struct
+
 import numpy as np
 import pytest
 
@@ -90,6 +94,25 @@ def test_resident_cg_gives_up_to_launch_chain(x, monkeypatch, shape):
     a = _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_PERSIST_WAIT_US="0")
     _same(a, _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_NO_PERSIST="1"))
     assert a[1][1:] == (1, 1, 0)
+
+
+def test_resident_cg_without_room_runs_the_launch_chain(x, monkeypatch):
+    """Compute units that another process holds (a lock on the device's file,
+    taken here through an open file of the test's own) are not waited for."""
+    mesh = _mesh(x, (131, 67))
+    free = _solve(x, mesh, x._abi.PREC_FP64, monkeypatch)
+    assert free[1][1:] == (2, 0, 0)
+    files = [open(f, "r+b") for f in glob.glob("/dev/shm/xcal-resident-*")]
+    assert files
+    for f in files:
+        fcntl.fcntl(f, fcntl.F_OFD_SETLK, struct.pack("hhqqi4x", fcntl.F_WRLCK, 0, 0, 64, 0))
+    held = _solve(x, mesh, x._abi.PREC_FP64, monkeypatch)
+    for f in files:
+        f.close()
+    assert held[1][1:] == (0, 0, 2)
+    _same(free, _solve(x, mesh, x._abi.PREC_FP64, monkeypatch, XCAL_NO_PERSIST="1"))
+    for u, v in zip(free[0], held[0]):
+        assert u[:3] == v[:3] and np.array_equal(u[3], v[3])
 
 
 def _batch(x, sizes, prec, monkeypatch, **env):

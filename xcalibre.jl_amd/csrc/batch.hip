@@ -1021,7 +1021,7 @@ static void bcg(BSolver<T>& S, int precon, const T* b, T* x0, int itmax, double 
   bool resident = false;
   if (!dilu && !graphs_enabled(c)) {  // the whole solve in one resident launch (persist.h)
     F.flush();
-    PersistLease lease;
+    ResidentLease lease;
     resident = persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease);
     if (resident && !bread(S)) {  // waits given up: start over by launches
       persist_failed(S.m);

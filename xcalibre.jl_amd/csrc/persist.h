@@ -24,8 +24,8 @@
 // below).
 //
 // All workgroups must be resident at once.  The host launches at most one
-// workgroup per compute unit over all solves in flight in the process
-// (PersistLease::acquire), and every wait is bounded in time: past the bound a
+// workgroup per compute unit over all solves in flight on the device
+// (ResidentRoom), and every wait is bounded in time: past the bound a
 // workgroup raises the abort word, marks its case's state and returns without
 // its rows of x, and so does each one that then waits in vain.  At the last
 // meeting the others may still find every sum and finish, so the host takes a

@@ -1,6 +1,6 @@
 // Resident CG (persist.h): workgroup plans, admission and launch.
-#include <atomic>
 #include <cstdlib>
+#include <mutex>
 
 #include "persist.h"
 
@@ -37,25 +37,20 @@ static int compute_units(int device) {
   return cu;
 }
 
-// Resident workgroups in flight per device, over every stream and thread of
-// the process: a launch is admitted only while all of them fit the device
-// one per compute unit, so admitted launches can never wait for each other.
-static std::atomic<int> g_resident[64];
-
-bool PersistLease::acquire(int device, int nwg, int cap) {
-  if (device < 0 || device >= 64) return false;
-  int cur = g_resident[device].load();
-  while (cur + nwg <= cap)
-    if (g_resident[device].compare_exchange_weak(cur, cur + nwg)) {
-      dev = device;
-      n = nwg;
-      return true;
-    }
-  return false;
-}
-void PersistLease::release() {
-  if (n > 0) g_resident[dev].fetch_sub(n);
-  n = 0;
+// Room for resident workgroups on each device (resident.h).  A launch is
+// admitted only while all in flight fit the device one per compute unit, so
+// admitted launches can never wait for each other.  The file that processes
+// share is named by the device's PCI address.
+static ResidentRoom* resident_room(int device) {
+  static ResidentRoom rooms[64];
+  static std::once_flag named[64];
+  if (device < 0 || device >= 64) return nullptr;
+  std::call_once(named[device], [&] {
+    char id[64] = {};
+    if (hipDeviceGetPCIBusId(id, sizeof id, device) == hipSuccess && id[0])
+      rooms[device].share(std::string("/dev/shm/xcal-resident-") + id);
+  });
+  return &rooms[device];
 }
 
 // Groups of 64 rows, the slots both reductions add them in, and the
@@ -148,13 +143,14 @@ static __global__ void __launch_bounds__(kBlock)
 // mesh on the launch chain from then on.
 template <class T>
 bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T* z, KS* ks,
-                PersistLease& lease) {
+                ResidentLease& lease) {
   const xcal_mesh* m = e->mesh;
   if (!m->persist_on || m->ctx->prof_on[0]) return false;
   if (!m->persist) m->persist = make_plan(m);
   const PersistPlan& P = *m->persist;
   if (!P.ok) return false;
-  if (!lease.acquire(m->ctx->device, P.nwg, compute_units(m->ctx->device))) {
+  ResidentRoom* room = resident_room(m->ctx->device);
+  if (!room || !lease.acquire(*room, P.nwg, compute_units(m->ctx->device))) {
     m->persist_full++;
     return false;
   }
@@ -187,9 +183,9 @@ bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T*
   return true;
 }
 template bool persist_cg<double>(xcal_eqn*, const MatKT<double>&, const double*, double*,
-                                 const double*, double*, KS*, PersistLease&);
+                                 const double*, double*, KS*, ResidentLease&);
 template bool persist_cg<float>(xcal_eqn*, const MatKT<float>&, const float*, float*, const float*,
-                                float*, KS*, PersistLease&);
+                                float*, KS*, ResidentLease&);
 
 void persist_failed(const xcal_mesh* m) {
   m->persist_on = false;

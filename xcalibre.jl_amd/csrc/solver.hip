@@ -1221,7 +1221,7 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
   }
   KS st{};
   if (!dilu) {  // small meshes: the whole solve in one resident launch (persist.h)
-    PersistLease lease;
+    ResidentLease lease;
     if (persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease)) {
       st = read_state(S);
       if (!resident_done(st.stop, st.gave_up)) {  // waits given up: start over by launches

@@ -417,20 +417,9 @@ __device__ inline void bwd_row(const BwdK<T>& W, int32_t pos, int64_t e0, int32_
 
 
 // ------------------------------------------------------------ resident CG
-// Workgroups of resident launches in flight (persist.hip): held from the
-// launch until its stream has been waited for.
-struct PersistLease {
-  int dev = 0, n = 0;
-  bool acquire(int device, int nwg, int cap);
-  void release();
-  PersistLease() = default;
-  PersistLease(const PersistLease&) = delete;
-  PersistLease& operator=(const PersistLease&) = delete;
-  ~PersistLease() { release(); }
-};
 template <class T>
 bool persist_cg(xcal_eqn* e, const MatKT<T>& A, const T* S, T* x, const T* r, T* z, KS* ks,
-                PersistLease& lease);
+                ResidentLease& lease);
 void persist_failed(const xcal_mesh* m);
 
 // ----------------------------------------------------- kernel timing hook
