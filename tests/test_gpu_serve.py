@@ -148,6 +148,32 @@ def test_serve_admission_respects_budget(x):
     srv.close()
 
 
+def test_serve_footprint_counts_the_lean_sweeps(x, monkeypatch):
+    """A cavity 256 cells wide takes the lean sweeps as a batch, one 258 wide
+    does not: their footprints per cell differ by the lean tables (measured on
+    the mesh) and, for each of the two DILU equations, six values per row."""
+    from conftest import cavity_case
+
+    api, H = x.api, x.hip
+    per_cell, srv = [], H.Server(0, slots=1, max_iterations=1)
+    for n in (256, 258):
+        mesh = x.mesh.cavity2d(n)
+        model, config = cavity_case(api, mesh, iterations=1)
+        rid = srv.submit(mesh, api.simple_setup(model, config, pref=0.0))
+        assert srv.wait(rid, 120.0)
+        per_cell.append(srv.status(rid)["footprint"] / mesh.n_cells)
+    srv.close()
+    ctx = api._context(0)
+    meshes = [x.mesh.cavity2d(256)]
+    dm = H.DeviceMesh.batch(ctx, meshes)
+    monkeypatch.setenv("XCAL_NO_PIPE", "1")
+    plain = H.DeviceMesh.batch(ctx, meshes)
+    assert dm.lean_form() == (4096, 4096) and plain.lean_form() == (0, 0)
+    tables = (dm.device_bytes - plain.device_bytes) / dm.n
+    # 16 bytes less: the rest of the estimate differs a little per cell
+    assert per_cell[0] - per_cell[1] >= tables + 2 * 6 * 8 - 16
+
+
 def test_serve_rejects_oversized_case(x):
     H = x.hip
     case = _case(x, 0.5, 2500, rans=False)

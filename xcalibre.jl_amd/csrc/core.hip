@@ -1336,6 +1336,25 @@ std::shared_ptr<PreparedMesh> prepare_union(const std::vector<const PreparedMesh
 
 int64_t prepared_cells(const PreparedMesh& P) { return P.U.n; }
 
+// Device bytes of the lean sweeps a batch of this case may build
+// (build_lean): per position w nz slots and one or two ring words a direction,
+// and per DILU equation a_ij of both triangles, the diagonal update's products
+// and one FP32 copy.  0 where its levels or rows are too wide for them.
+static int64_t lean_footprint(const HostMesh& M, int equations) {
+  int w[2] = {2, 2};
+  const std::vector<int32_t>* ptr[2] = {&M.lev_ptr_f, &M.lev_ptr_b};
+  const std::vector<int32_t>* meta[2] = {&M.lmeta_f, &M.lmeta_b};
+  for (int d = 0; d < 2; ++d)
+    for (size_t l = 0; l + 1 < ptr[d]->size(); ++l) {
+      if ((*ptr[d])[l + 1] - (*ptr[d])[l] > kPipeBlock) return 0;
+      w[d] = std::max(w[d], (*meta[d])[2 * l + 1]);
+    }
+  if (std::max(w[0], w[1]) > kLeanWidth) return 0;
+  const int64_t both = w[0] + w[1], steps = 8 * (M.lev_ptr_f.size() + M.lev_ptr_b.size());
+  return M.n * (4 * both + 4 * (w[0] - 1) + 4 * (w[1] - 1) +
+                equations * 8 * (both + w[0]) + 4 * both) + steps;
+}
+
 // Device bytes of a prepared mesh plus a steady SIMPLE run on it (fields,
 // the U and p equations with DILU, FP64 and FP32 Krylov workspaces).
 int64_t prepared_footprint(const PreparedMesh& P, bool turb) {
@@ -1352,7 +1371,7 @@ int64_t prepared_footprint(const PreparedMesh& P, bool turb) {
   const int64_t eqns = 8 * (3 * nz + 4 * n) + 8 * 2 * (nz + 3 * n);
   const int64_t krylov = 2 * 8 * 12 * n + 4 * (12 * n + nz + 3 * n);
   const int64_t turbulence = turb ? 8 * (8 * n + 3 * nf) : 0;
-  return mesh + fields + eqns + krylov + turbulence;
+  return mesh + fields + eqns + krylov + turbulence + lean_footprint(M, turb ? 4 : 2);
 }
 
 // Lean form of one sweep direction (sweep_lean.h): steps of at most
