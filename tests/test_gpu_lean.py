@@ -6,8 +6,9 @@ the reference's summation order and the dot products the launch form's, so
 preconditioner applies, CG and BiCGSTAB solves equal those of XCAL_NO_PIPE=1
 (level launches and level-stepping runs) exactly.  Shapes: level counts on
 both sides of a multiple of the step padding, levels of one row up to several
-steps, two and three entries per row, and dependencies that need the longer
-LDS ring."""
+steps, two and three entries per row, dependencies that need the longer LDS
+ring, and long meshes above the cone form's size, whose levels are too many
+for bands."""
 import numpy as np
 import pytest
 
@@ -58,7 +59,7 @@ def _setup(A, solver, prec):
 
 
 SHAPES = [(9, 8), (9, 9), (40, 1), (23, 18), (63, 37), (130, 260), (200, 255), (5, 6, 7),
-          (16, 17, 18), (37, 21, 29), ("step", 24), ("step", 104)]
+          (16, 17, 18), (37, 21, 29), ("step", 24), ("step", 104), (1000, 90), (600, 12, 12)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)

@@ -1,7 +1,9 @@
 // Context, mesh upload and fields of libxcalhip.so.
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <memory>
 #include <numeric>
 
@@ -344,24 +346,21 @@ static bool build_band(int S, double ratio, bool lower, const std::vector<int32_
 }
 
 // Builds the cone form of the forward (lower) or backward (upper) sweep with
-// blocks of S rows over nlev levels.  First every level as one band; where
-// those cones do not fit, bands of consecutive levels, each launch then
+// blocks of S rows over nlev levels: every level as one band (bratio 0), or,
+// where those cones do not fit, bands of consecutive levels, each launch then
 // covering only the band's rows: a band's block size is the power of two
 // (kConeMinBlock..S) that gives about kConeBandBlocks blocks, so a launch
-// still fills the chip, doubled while its cone positions exceed
-// kConeBandRatio times its rows (larger blocks recompute fewer rows; fewer,
-// wider bands pay for more recomputed rows: PISO on 308k naturally numbered
-// cells 160, 141, 135, 127, 125 ms at ratios 2, 3, 4, 6, 8, 85k cells 45.9,
-// 40.3, 39.2, 36.3, 36.1, and 8 holds a third more positions than 6).  A
-// band starts at twice the previous band's width (the levels left, for the
-// first) and halves when no block size fits.  False
-// when a band of kConeMinBand levels does not fit, the sweep needs more than
-// kConeMaxBands bands, or the cones hold more than kConeMaxRatio n
-// positions in all.
+// still fills the chip, doubled while its cone positions exceed bratio times
+// its rows (larger blocks recompute fewer rows).  A band starts at twice the
+// previous band's width (the levels left, for the first) and halves when no
+// block size fits.  False when a band of kConeMinBand levels does not fit, the
+// sweep needs more than kConeMaxBands bands, the cones hold more than
+// kConeMaxRatio n positions in all, or `cancel` was set.
 static bool build_cone(int64_t n, int S, bool lower, const std::vector<int32_t>& ord,
                        const std::vector<int32_t>& lev, int nlev, const std::vector<int32_t>& rbeg,
                        const std::vector<int32_t>& rend, const std::vector<int32_t>& diag,
-                       const std::vector<int32_t>& colval, ConeHost& C) {
+                       const std::vector<int32_t>& colval, double bratio,
+                       const std::atomic<bool>& cancel, ConeHost& C) {
   C = ConeHost();
   C.blk.push_back(0);
   C.base.push_back(0);
@@ -371,16 +370,17 @@ static bool build_cone(int64_t n, int S, bool lower, const std::vector<int32_t>&
   std::vector<int64_t> lcnt(nlev + 1, 0);  // rows below each level
   for (int64_t c = 0; c < n; ++c) lcnt[lev[c] + 1]++;
   for (int l = 0; l < nlev; ++l) lcnt[l + 1] += lcnt[l];
-  double bratio = kConeBandRatio;  // XCAL_CONE_BAND_RATIO at creation overrides it
-  if (const char* env = std::getenv("XCAL_CONE_BAND_RATIO")) bratio = std::max(1.0, std::atof(env));
   const double maxratio = std::max(kConeMaxRatio, bratio + 0.5);
   int lo = 0, H = nlev;
-  if (build_band(S, 0, lower, ord, lev, 0, nlev, rbeg, rend, diag, colval, C, W)) {
+  if (bratio == 0) {
+    if (!build_band(S, 0, lower, ord, lev, 0, nlev, rbeg, rend, diag, colval, C, W) ||
+        (double)C.crow.size() > kConeMaxRatio * (double)n)
+      return false;
     C.band.push_back((int32_t)C.blk.size() - 1);
     lo = nlev;
-    if ((double)C.crow.size() > kConeMaxRatio * (double)n) return false;
   }
   while (lo < nlev) {
+    if (cancel) return false;
     H = std::min(H, nlev - lo);
     for (;;) {
       const int64_t rows = lcnt[lo + H] - lcnt[lo];
@@ -858,12 +858,47 @@ static void build_host_mesh(const xcal_mesh_host* h, HostMesh& M, bool cones, xc
     }
     std::stable_sort(ord.begin(), ord.end(),
                      [&](int32_t a, int32_t b) { return dmort[a] < dmort[b]; });
+    const char* fixed = std::getenv("XCAL_CONE_BAND_RATIO");
+    const double ratio = fixed ? std::max(1.0, std::atof(fixed)) : kConeBandRatio;
+    // Meshes with more than 2.5 entries per row and triangle (hexahedra have
+    // three, quadrilaterals two) that take bands have them with kConeWideRatio.
+    const bool wide = !fixed && (double)(nnz - n) > 2 * 2.5 * (double)n;
+    struct Cones {
+      bool ok = false, wide = false;
+      ConeHost c, w;
+    };
+    // both sweeps' cones, and both kinds of bands, at once
+    auto build = [&](int S, bool lower, std::atomic<bool>& cancel) {
+      Cones t;
+      auto make = [&](double most, ConeHost& C) {
+        return lower ? build_cone(n, S, true, ord, flev_d, M.nlev_f, rbeg, rend, diag_n, colval_n,
+                                  most, cancel, C)
+                     : build_cone(n, S, false, ord, blev_d, M.nlev_b, rbeg, rend, diag_n, colval_n,
+                                  most, cancel, C);
+      };
+      t.ok = make(0, t.c);
+      if (t.ok) return t;
+      if (t.c.blk.size() > 1) {  // one band fits the blocks with too many positions
+        cancel = true;
+        return t;
+      }
+      std::future<bool> w;
+      if (wide) w = std::async(std::launch::async, [&] { return make(kConeWideRatio, t.w); });
+      t.ok = make(ratio, t.c);
+      if (!t.ok) cancel = true;
+      t.wide = w.valid() && w.get();
+      return t;
+    };
     for (int S = rows; S >= 64 && !M.cone; S /= 2) {
-      M.cone = build_cone(n, S, true, ord, flev_d, M.nlev_f, rbeg, rend, diag_n, colval_n,
-                          M.cone_f) &&
-               build_cone(n, S, false, ord, blev_d, M.nlev_b, rbeg, rend, diag_n, colval_n,
-                          M.cone_b);
-      if (M.cone) M.cone_rows = S;
+      std::atomic<bool> cancel{false};
+      auto back = std::async(std::launch::async, [&] { return build(S, false, cancel); });
+      Cones F = build(S, true, cancel), B = back.get();
+      M.cone = F.ok && B.ok;
+      if (M.cone) {
+        M.cone_rows = S;
+        M.cone_f = std::move(F.wide ? F.w : F.c);
+        M.cone_b = std::move(B.wide ? B.w : B.c);
+      }
       if (S <= 256) break;
     }
     if (!M.cone) M.cone_f = M.cone_b = ConeHost();

@@ -94,7 +94,16 @@ constexpr int kConeMinBand = 4;            // narrowest band of levels
 constexpr int kConeMaxBands = 128;         // most bands (launches) per sweep
 constexpr int kConeMinBlock = 64;          // smallest block of a band
 constexpr int kConeBandBlocks = 512;       // blocks a band's block size aims at
-constexpr double kConeBandRatio = 6.0;     // most cone positions per row of a band
+// Most cone positions per row of a band.  kConeBandRatio decides whether a
+// mesh takes bands at all: long meshes do not at 4 and would at 6, where one
+// workgroup's sweep is the faster (per apply 1000x90 quadrilaterals 422 us
+// against 1043, 600x12x12 hexahedra 277 against 779).  kConeWideRatio is what
+// hexahedral bands are then made with (per apply and per CG iteration in FP64,
+// 4 then 6: 79x66x59 cells 440 to 415 and 397 to 366 us, 300x120x6 823 to 674
+// and 709 to 619; 260x260 quadrilaterals would go from 425 to 454 and from 485
+// to 500; 8 holds a third more positions than 6 for 1%).
+constexpr double kConeBandRatio = 4.0;
+constexpr double kConeWideRatio = 6.0;
 constexpr int kSplitDepth = 4;  // steps in flight of the split CG's sweeps (and their padding)
 
 // Lean one-workgroup sweeps (sweep_lean.h): threads, prefetch depth (and
