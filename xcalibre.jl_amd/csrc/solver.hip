@@ -1138,10 +1138,13 @@ static KS cg_split(Solver<T>& S, T* w) {
   KS* cur = S.ks;
   auto other = [&](KS* k) { return k == S.ks ? S.fks : S.ks; };
   auto fwd = [&](auto start, const T* u, T* out) {
-    for (size_t k = 0; k + 1 < bf.size(); ++k)
-      hipLaunchKernelGGL((k_split_fwd<decltype(start)::value, T>), dim3(bf[k + 1] - bf[k]),
-                         dim3(kConeBlock), 0, S.s, split_k(m->cone_f, bf[k]), f.a, f.f, u,
-                         (const T*)t, out, wv, n, p0, (const KS*)cur);
+    with_split_pairs(m->cone_f, [&](auto J) {
+      for (size_t k = 0; k + 1 < bf.size(); ++k)
+        hipLaunchKernelGGL((k_split_fwd<decltype(start)::value, decltype(J)::value, T>),
+                           dim3(bf[k + 1] - bf[k]), dim3(kConeBlock), 0, S.s,
+                           split_k(m->cone_f, bf[k]), f.a, f.f, u, (const T*)t, out, wv, n, p0,
+                           (const KS*)cur);
+    });
   };
   fwd(std::true_type{}, (const T*)u0, rho);
   finalize_launch(S, nf, FIN_CG_INIT);
@@ -1155,10 +1158,12 @@ static KS cg_split(Solver<T>& S, T* w) {
     const KStep Kb{cur, other(cur), p1, vg, pend ? FIN_CG_ITER : FIN_NONE};
     const KStep Kn = kstep_plain(other(cur));
     timed(m->ctx, 2, [&] {
-      for (size_t k = 0; k + 1 < bb.size(); ++k)
-        hipLaunchKernelGGL(k_split_bwd<T>, dim3(bb[k + 1] - bb[k]), dim3(kConeBlock), 0, S.s,
-                           split_k(m->cone_b, bb[k]), f.b, f.d, (const T*)rho, (const T*)pold, pnew,
-                           t, n, k == 0 ? Kb : Kn);
+      with_split_pairs(m->cone_b, [&](auto J) {
+        for (size_t k = 0; k + 1 < bb.size(); ++k)
+          hipLaunchKernelGGL((k_split_bwd<decltype(J)::value, T>), dim3(bb[k + 1] - bb[k]),
+                             dim3(kConeBlock), 0, S.s, split_k(m->cone_b, bb[k]), f.b, f.d,
+                             (const T*)rho, (const T*)pold, pnew, t, n, k == 0 ? Kb : Kn);
+      });
     });
     cur = other(cur);
     timed(m->ctx, 1, [&] { fwd(std::false_type{}, (const T*)pnew, q); });

@@ -20,10 +20,12 @@
 // steps), with each row's loads packed: one 16-byte record (device row, six
 // 16-bit cone positions), its entries in pairs (a step's rows are ordered by
 // entry count, so pair j holds rows [0, pcnt[j])), and its scalars; a missing
-// entry reads an LDS slot that holds 0.  Seven loads and about 60 issued
-// instructions per row and step against 16 and 110, the dependencies read
-// from LDS together instead of one after the other, and half the LDS per
-// block.  Stores of rows that another block owns are dropped by the buffer
+// entry reads an LDS slot that holds 0.  A kernel takes as many pairs as the
+// sweep's longest row: one on naturally numbered quadrilaterals, two on
+// hexahedra, three on randomly numbered hexahedra.  With three pairs seven
+// loads and about 60 issued instructions per row and step against 16 and 110,
+// the dependencies read from LDS together instead of one after the other, and
+// half the LDS per block.  Stores of rows that another block owns are dropped by the buffer
 // store's range check instead of a branch, which would end the loop's block
 // and with it exact waits.
 //
@@ -39,7 +41,8 @@
 // classical (35 + 32 + 27 + 8), 87 split in device order (48 backward, 27
 // forward, 12 vectors), 66 in block order (28 + 26 + 11); 343k random box
 // 66, 43 and 40; 152k random box in FP32 57, 33 and 31; 308k natural box
-// (bands) 530 and 420.  Both sweeps are bound by the step-to-step chain and
+// (bands, two pairs) 500 and 346; 67.6k-cell cavity (bands, one pair) in FP64
+// 505 and 413, in FP32 403 and 343 (three pairs 482 and 437).  Both sweeps are bound by the step-to-step chain and
 // the 1.75 n rows of the cones; 4 steps in flight, 6 and 5 were no faster.
 #pragma once
 
@@ -81,24 +84,27 @@ struct OwnStore {
   }
 };
 
-// A row of a step: record, entry pairs and scalars in flight.
-template <class T, int NS>
+// A row of a step: record (J = 1: its first half), entry pairs and scalars in
+// flight.
+template <class T, int NS, int J>
 struct SplitRec {
-  int4 rec;
-  T a[6], sc[NS], g0, g1;
+  int row;
+  uint32_t w[J];
+  T a[2 * J], sc[NS], g0, g1;
   uint32_t lp;
   bool in;
 };
 
-// Walks block b's steps.  NS scalars per position at `sc`; g0 and, with NG = 2,
+// Walks block b's steps.  J entry pairs per row (the most that one has); NS
+// scalars per position at `sc`; g0 and, with NG = 2,
 // g1 are gathered from G0 and G1 by row; work(R, row, sum) returns the row's
 // value.  Halo values come from `halo`.
-template <int NS, int NG, class T, class Work>
+template <int J, int NS, int NG, class T, class Work>
 __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ a,
                                   const T* __restrict__ sc, const T* __restrict__ halo,
                                   const T* __restrict__ G0, const T* __restrict__ G1, T* v,
                                   Work&& work) {
-  using R = SplitRec<T, NS>;
+  using R = SplitRec<T, NS, J>;
   constexpr int P = kSplitDepth, Q = kSplitGather;
   const int s0 = C.blk[b], ns = C.blk[b + 1] - s0;
   const int32_t base = C.base[b], nh = C.hnum[b];
@@ -107,21 +113,38 @@ __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ 
   __syncthreads();
   const auto* words = (const __attribute__((address_space(4))) int32_t*)(C.step + 8 * (int64_t)s0);
   struct Step {
-    int32_t r0, cnt, po[3], pc[3];
+    int32_t r0, cnt, po[J], pc[J];
   };
   auto step = [&](int l) {
     const int o = 8 * min(l, ns - 1);
-    return Step{words[o],     words[o + 1], {words[o + 2], words[o + 3], words[o + 4]},
-                {words[o + 5], words[o + 6], words[o + 7]}};
+    Step t;
+    t.r0 = words[o];
+    t.cnt = words[o + 1];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      t.po[j] = words[o + 2 + j];
+      t.pc[j] = words[o + 5 + j];
+    }
+    return t;
   };
   typedef T V2 __attribute__((ext_vector_type(2)));
   auto fetch = [&](R& r, const Step& st) {
     const uint32_t q = min((uint32_t)threadIdx.x, (uint32_t)max(st.cnt, 1) - 1u);
     const uint32_t pos = (uint32_t)st.r0 + q;
     r.in = (int)threadIdx.x < st.cnt;
-    r.rec = lean_at<int4>(C.rec, pos);
+    if constexpr (J == 1) {
+      const int2 u = lean_at<int2>(C.rec, 2 * pos);
+      r.row = u.x;
+      r.w[0] = (uint32_t)u.y;
+    } else {
+      const int4 u = lean_at<int4>(C.rec, pos);
+      r.row = u.x;
+      r.w[0] = (uint32_t)u.y;
+      r.w[1] = (uint32_t)u.z;
+      if constexpr (J == 3) r.w[2] = (uint32_t)u.w;
+    }
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
+    for (int j = 0; j < J; ++j) {
       const V2 p = lean_at<V2>(a, (int)q < st.pc[j] ? (uint32_t)st.po[j] + q : 0u);
       r.a[2 * j] = p.x;
       r.a[2 * j + 1] = p.y;
@@ -135,30 +158,28 @@ __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ 
     }
     r.lp = pos - (uint32_t)base;
   };
-  auto row = [](const R& r) { return (uint32_t)(r.rec.x ^ (r.rec.x >> 31)); };
+  auto row = [](const R& r) { return (uint32_t)(r.row ^ (r.row >> 31)); };
   auto gather = [&](R& r) {
-    opaque(r.rec.x);
+    opaque(r.row);
     r.g0 = lean_at<T>(G0, row(r));
     if constexpr (NG == 2) r.g1 = lean_at<T>(G1, row(r));
   };
   auto process = [&](R& r) {
-    opaque(r.rec.x);
-    opaque(r.rec.y);
-    opaque(r.rec.z);
-    opaque(r.rec.w);
+    opaque(r.row);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) opaque(r.a[k]);
+    for (int j = 0; j < J; ++j) opaque(r.w[j]);
+#pragma unroll
+    for (int k = 0; k < 2 * J; ++k) opaque(r.a[k]);
 #pragma unroll
     for (int k = 0; k < NS; ++k) opaque(r.sc[k]);
     opaque(r.g0);
     if constexpr (NG == 2) opaque(r.g1);
-    const uint32_t w[3] = {(uint32_t)r.rec.y, (uint32_t)r.rec.z, (uint32_t)r.rec.w};
-    T d[6];
+    T d[2 * J];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) d[k] = v[k & 1 ? w[k >> 1] >> 16 : w[k >> 1] & 0xffff];
+    for (int k = 0; k < 2 * J; ++k) d[k] = v[k & 1 ? r.w[k >> 1] >> 16 : r.w[k >> 1] & 0xffff];
     T sum = 0;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) sum = sum + r.a[k] * d[k];
+    for (int k = 0; k < 2 * J; ++k) sum = sum + r.a[k] * d[k];
     v[r.lp] = work(r, row(r), sum);
   };
   R buf[P];
@@ -181,7 +202,7 @@ __device__ inline void split_walk(const SplitK& C, int b, const T* __restrict__ 
 
 // Backward sweep: the pending rho.rho/D finalize (kstate; every workgroup),
 // then ph = rho + beta pold, t = (D + U)^-1 ph.
-template <class T>
+template <int J, class T>
 __global__ void __launch_bounds__(kConeBlock)
     k_split_bwd(SplitK C, const T* __restrict__ a, const T* __restrict__ rD,
                 const T* __restrict__ rho, const T* __restrict__ pold, T* __restrict__ ph, T* t,
@@ -192,11 +213,11 @@ __global__ void __launch_bounds__(kConeBlock)
   if (k.stop != STOP_NONE) return;  // uniform over the grid
   const T beta = (T)k.beta;
   const OwnStore<T> sp(ph, n), st(t, n);
-  split_walk<1, 2, T>(C, C.blk0 + (int)xcd_block(), a, rD, (const T*)t, rho, pold, v,
-                   [&](const SplitRec<T, 1>& r, uint32_t i, T sum) {
+  split_walk<J, 1, 2, T>(C, C.blk0 + (int)xcd_block(), a, rD, (const T*)t, rho, pold, v,
+                   [&](const SplitRec<T, 1, J>& r, uint32_t i, T sum) {
                      const T p = r.g0 + beta * r.g1;
                      const T z = (p - sum) * r.sc[0];
-                     const bool own = r.rec.x >= 0;
+                     const bool own = r.row >= 0;
                      sp.put(own, i, p);
                      st.put(own, i, z);
                      return z;
@@ -208,7 +229,7 @@ __global__ void __launch_bounds__(kConeBlock)
 // only where a later band reads it as its halo (w may be null otherwise).
 // START: u = ph given alone; rho = y = u - sum a_ij w_j, w = y / D,
 // partials of rho.rho/D.
-template <bool START, class T>
+template <bool START, int J, class T>
 __global__ void __launch_bounds__(kConeBlock)
     k_split_fwd(SplitK C, const T* __restrict__ a, const T* __restrict__ sc,
                 const T* __restrict__ ph, const T* __restrict__ t, T* __restrict__ q, T* w,
@@ -218,9 +239,9 @@ __global__ void __launch_bounds__(kConeBlock)
   const int b = C.blk0 + (int)xcd_block();
   const OwnStore<T> sq(q, n), sw(w, w ? n : 0);
   double s0 = 0.0;
-  split_walk<2, START ? 1 : 2, T>(C, b, a, sc, (const T*)w, ph, t, v,
-                   [&](const SplitRec<T, 2>& r, uint32_t i, T sum) {
-                     const bool own = r.rec.x >= 0;
+  split_walk<J, 2, START ? 1 : 2, T>(C, b, a, sc, (const T*)w, ph, t, v,
+                   [&](const SplitRec<T, 2, J>& r, uint32_t i, T sum) {
+                     const bool own = r.row >= 0;
                      T wi, qi, qd;
                      if (START) {
                        qi = r.g0 - sum;
@@ -278,6 +299,13 @@ __global__ void __launch_bounds__(kBlock)
   store_partial<kBlock>(s0, 0.0, partial, blockIdx.x);
 }
 
+// Host: calls f(J) with the entry pairs of a cone's rows.
+template <class F>
+inline void with_split_pairs(const xcal_mesh::Cone& c, F&& f) {
+  if (c.wk <= 2) f(std::integral_constant<int, 1>{});
+  else if (c.wk <= 4) f(std::integral_constant<int, 2>{});
+  else f(std::integral_constant<int, 3>{});
+}
 // Host: the kernel view of one direction's tables for the band from blk0.
 inline SplitK split_k(const xcal_mesh::Cone& c, int32_t blk0) {
   return SplitK{c.step2.p, c.blk2.p, c.base.p, c.hnum.p, c.rec.p, blk0};
