@@ -93,3 +93,47 @@ def test_split_cg_stops_at_itmax(x, A, ctx, monkeypatch, itmax):
     for u, v in zip(a, b):
         assert u[0] == v[0] == itmax and u[1] == v[1] == 1
         assert rel(u[2], v[2]) < 1e-12  # a few iterations' rounding
+
+
+@pytest.mark.parametrize("prec", ["PREC_FP64", "PREC_FP32_IR"])
+def test_split_cg_follows_the_matrix_from_update_to_update(x, A, ctx, monkeypatch, prec):
+    """One equation whose matrix is made symmetric and not by turns, on a mesh
+    with and without the split form: solves of the nonsymmetric ones, also those
+    that had started in the split form, and of a single iteration are the
+    classical ones bit for bit, the others agree as above and are not."""
+    H = x.hip
+    mesh = _mesh(x, "random")
+    runs = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("XCAL_NO_SPLIT", "1")
+        dm = H.DeviceMesh(ctx, mesh)
+        monkeypatch.delenv("XCAL_NO_SPLIT", raising=False)
+        rng = np.random.default_rng(8)
+        g = H.Field(dm, A.FACE_SCALAR).upload(0.5 + rng.random(mesh.n_faces))
+        md = H.Field(dm, A.FACE_SCALAR).upload(1e-3 * rng.standard_normal(mesh.n_faces))
+        s = H.Field(dm, A.CELL_SCALAR).upload(rng.standard_normal(mesh.n_cells))
+        start = rng.standard_normal(mesh.n_cells)
+        bcs = A.bc_array([(A.BC_DIRICHLET if i == 0 else A.BC_ZEROGRADIENT, i, 0.0)
+                          for i in range(len(mesh.patch_names))])
+        eq, phi = H.Equation(dm, False), H.Field(dm, A.CELL_SCALAR)
+        out = []
+        for kind, itmax in (("sym", 12), ("asym", 12), ("asym", 12), ("sym", 12), ("sym", 1),
+                            ("asym", 12), ("sym", 12)):
+            terms = [(A.LAPLACIAN_LINEAR, -1, g)]
+            terms += [(A.DIV_UPWIND, 1, md)] if kind == "asym" else []
+            phi.upload(start)
+            eq.discretise(terms, [(s, 1)])
+            eq.apply_bcs(terms, bcs, phi)
+            eq.precond_update(A.PRECON_DILU)
+            n, _, rc = eq.solve(A.SolverSetupC(A.SOLVER_CG, A.PRECON_DILU, getattr(A, prec), itmax,
+                                               1e-7, 1.0, 1e-14, 1e-10, 1e-6, 0, 0.0), phi)
+            out.append((kind, itmax, n, rc, phi.download()))
+        runs.append(out)
+    for u, v in zip(*runs):
+        assert u[:4] == v[:4]
+        if u[0] == "asym" or u[1] == 1:
+            assert np.array_equal(u[4], v[4])
+        else:  # twelve iterations' rounding, in the sweeps' precision
+            assert rel(u[4], v[4]) < (1e-12 if prec == "PREC_FP64" else 1e-4)
+            assert not np.array_equal(u[4], v[4])

@@ -140,18 +140,19 @@ __global__ void __launch_bounds__(kConeBlock)
   __shared__ ConeLDS<double> L;
   diag_cone<WK, P>(C, prod, ajj, D, L);
 }
-__global__ void k_clear_flag(int32_t* flag) { *flag = 0; }
+__global__ void k_clear_stamp(int32_t* p) { *p = 0; }
 // a_ji a_ij per cone entry (0 where the transpose is absent, which a face
-// matrix's symmetric pattern never has), and a_ij itself
+// matrix's symmetric pattern never has), and a_ij itself; *asym becomes this
+// update's stamp where the two differ
 __global__ void __launch_bounds__(kBlock)
     k_cone_products(int64_t n, const int32_t* __restrict__ slot, const int32_t* __restrict__ trans,
                     const double* __restrict__ nz, double* __restrict__ out,
-                    double* __restrict__ a, int32_t* asym) {
+                    double* __restrict__ a, int32_t* asym, int32_t stamp) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n) return;
   const int32_t k = slot[e], kt = trans[k];
   const double aij = nz[k];
-  if (kt < 0 || !(nz[kt] == aij)) *asym = 1;  // every writer stores the same
+  if (kt < 0 || !(nz[kt] == aij)) *asym = stamp;  // every writer stores the same
   out[e] = kt >= 0 ? nz[kt] * aij : 0.0;
   a[e] = aij;
 }
@@ -310,11 +311,13 @@ void precond_update(xcal_eqn* e, int precon) {
       }
       hipLaunchKernelGGL(k_gather_cone_rows, dim3(grid_for(F.rows)), dim3(kBlock), 0, s, F.rows,
                          F.crow.p, e->pD.p, e->cfd.p);
-      if (e->asym.n < 1) e->asym.alloc(1);
-      hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, s, e->asym.p);
+      if (e->asym.n < 1) {
+        e->asym.alloc(1);
+        hipLaunchKernelGGL(k_clear_stamp, dim3(1), dim3(1), 0, s, e->asym.p);
+      }
       hipLaunchKernelGGL(k_cone_products, dim3(grid_for(F.entries)), dim3(kBlock), 0, s,
                          F.entries, F.slot.p, m->trans.p, e->nzval.p, e->cfr.p, e->cfa.p,
-                         e->asym.p);
+                         e->asym.p, (int32_t)(e->precon_count + 1));
       with_cone_form(F.wk, !m->cone_deep, [&](auto WK, auto P) {
         for (size_t k = 0; k + 1 < F.band.size(); ++k)
           hipLaunchKernelGGL((k_dilu_diag_cone<decltype(WK)::value, decltype(P)::value>),
@@ -364,6 +367,7 @@ void precond_update(xcal_eqn* e, int precon) {
                          F.crow.p, e->prD.p, e->cfd.p);
       launch_check();
       e->precon_gen = e->nz_gen;
+      e->precon_count++;
       return;
     }
     if (m->pipe_wf > 0 || m->pipe_runs) {  // 1/D per packed lower entry, for the pipelined sweeps

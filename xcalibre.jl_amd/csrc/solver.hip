@@ -425,11 +425,12 @@ __global__ void __launch_bounds__(kBlock)
 
 // split CG factors: nz of each entry of the pairs (0 where there is none),
 // and out[p] = v of cone position p's row
+template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_split_pairs(int64_t n, const int32_t* __restrict__ slot, const double* __restrict__ nz,
-                  double* __restrict__ out) {
+                  T* __restrict__ out) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) out[e] = slot[e] >= 0 ? nz[slot[e]] : 0.0;
+  if (e < n) out[e] = slot[e] >= 0 ? (T)nz[slot[e]] : T(0);
 }
 template <class T>
 __global__ void __launch_bounds__(kBlock)
@@ -449,16 +450,17 @@ __global__ void __launch_bounds__(kBlock)
   out[i] = ADD ? out[i] + x[p] : x[p];
 }
 // (1/D, a_ii - D) per forward cone position
+template <class T>
 __global__ void __launch_bounds__(kBlock)
     k_split_scalars(int64_t total, const int32_t* __restrict__ crow,
                     const int32_t* __restrict__ diag, const double* __restrict__ nz,
                     const double* __restrict__ D, const double* __restrict__ rD,
-                    double* __restrict__ out) {
+                    T* __restrict__ out) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= total) return;
   const int32_t c = crow[p], i = c >= 0 ? c : ~c;
-  out[2 * p] = rD[i];
-  out[2 * p + 1] = nz[diag[i]] - D[i];
+  out[2 * p] = (T)rD[i];
+  out[2 * p + 1] = (T)(nz[diag[i]] - D[i]);
 }
 
 // b = 1 / a rounded to FP32
@@ -1017,44 +1019,43 @@ void precond_apply_staged(xcal_eqn* e, const double* r, double* z, double* Y, do
   dilu_apply(S, r, z, Y, Yb);
 }
 
-// The split CG's factors (sweep_split.h), made at a solve from the
-// preconditioner's: only CG on a symmetric matrix uses them.
+// The split CG's factors (sweep_split.h), made from the preconditioner's at
+// the first solve after its update that needs them: only CG on a symmetric
+// matrix does, the backward sweep's only once an iteration runs.
 template <class T>
-struct SplitFactors {
-  const T *a, *b, *f, *d;  // forward and backward pairs, (1/D, a_ii - D), 1/D
-};
-static SplitFactors<double> split_factors(xcal_eqn* e, double) {
+static void split_pairs(xcal_eqn* e, DBuf<T>& v, const DBuf<int32_t>& slot) {
+  if (v.n != slot.n) v.alloc(slot.n);
+  hipLaunchKernelGGL(k_split_pairs<T>, dim3(grid_for(slot.n)), dim3(kBlock), 0,
+                     e->mesh->ctx->stream, slot.n, slot.p, (const double*)e->nzval.p, v.p);
+}
+template <class T>
+static void split_factors_f(xcal_eqn* e, xcal_eqn::Split<T>& f) {
+  if (f.gen_f == e->precon_count) return;
   const xcal_mesh* m = e->mesh;
-  const xcal_mesh::Cone &F = m->cone_f, &B = m->cone_b;
-  hipStream_t s = m->ctx->stream;
-  auto pairs = [&](DBuf<double>& v, const DBuf<int32_t>& slot) {
-    if (v.n != slot.n) v.alloc(slot.n);
-    hipLaunchKernelGGL(k_split_pairs, dim3(grid_for(slot.n)), dim3(kBlock), 0, s, slot.n, slot.p,
-                       (const double*)e->nzval.p, v.p);
-  };
-  pairs(e->spa, F.pslot);
-  pairs(e->spb, B.pslot);
-  if (e->spf.n != 2 * F.rows) e->spf.alloc(2 * F.rows);
-  if (e->spd.n != B.rows) e->spd.alloc(B.rows);
-  hipLaunchKernelGGL(k_split_scalars, dim3(grid_for(F.rows)), dim3(kBlock), 0, s, F.rows, F.crow.p,
-                     m->diag.p, (const double*)e->nzval.p, (const double*)e->pD.p,
-                     (const double*)e->prD.p, e->spf.p);
-  hipLaunchKernelGGL(k_split_rows<double>, dim3(grid_for(B.rows)), dim3(kBlock), 0, s, B.rows, B.crow.p,
-                     (const double*)e->prD.p, e->spd.p);
+  const xcal_mesh::Cone& F = m->cone_f;
+  split_pairs(e, f.a, F.pslot);
+  if (f.f.n != 2 * F.rows) f.f.alloc(2 * F.rows);
+  hipLaunchKernelGGL(k_split_scalars<T>, dim3(grid_for(F.rows)), dim3(kBlock), 0, m->ctx->stream,
+                     F.rows, F.crow.p, m->diag.p, (const double*)e->nzval.p,
+                     (const double*)e->pD.p, (const double*)e->prD.p, f.f.p);
   XCAL_HIP(hipGetLastError());
-  return {e->spa.p, e->spb.p, e->spf.p, e->spd.p};
+  f.gen_f = e->precon_count;
 }
-static SplitFactors<float> split_factors(xcal_eqn* e, float) {
-  split_factors(e, 0.0);
-  hipStream_t s = e->mesh->ctx->stream;
-  auto cvt = [&](DBuf<float>& d, const DBuf<double>& a) {
-    if (d.n != a.n) d.alloc(a.n);
-    hipLaunchKernelGGL(k_to_float, dim3(grid_for(a.n)), dim3(kBlock), 0, s, a.n, a.p, d.p);
-    return (const float*)d.p;
-  };
-  return {cvt(e->spa32, e->spa), cvt(e->spb32, e->spb), cvt(e->spf32, e->spf),
-          cvt(e->spd32, e->spd)};
+// rD: the preconditioner's 1/D in T
+template <class T>
+static void split_factors_b(xcal_eqn* e, xcal_eqn::Split<T>& f, const T* rD) {
+  if (f.gen_b == e->precon_count) return;
+  const xcal_mesh* m = e->mesh;
+  const xcal_mesh::Cone& B = m->cone_b;
+  split_pairs(e, f.b, B.pslot);
+  if (f.d.n != B.rows) f.d.alloc(B.rows);
+  hipLaunchKernelGGL(k_split_rows<T>, dim3(grid_for(B.rows)), dim3(kBlock), 0, m->ctx->stream,
+                     B.rows, B.crow.p, rD, f.d.p);
+  XCAL_HIP(hipGetLastError());
+  f.gen_b = e->precon_count;
 }
+static xcal_eqn::Split<double>& split_of(xcal_eqn* e, double) { return e->split; }
+static xcal_eqn::Split<float>& split_of(xcal_eqn* e, float) { return e->split32; }
 
 template <class T>
 static KS read_state(Solver<T>& S) {
@@ -1098,32 +1099,56 @@ static int run_batches(Solver<T>& S, int* pred, int tail, const std::function<vo
   return out.stop;
 }
 
-// Whether a CG solve takes the split form: cone mesh with its tables, FP64 or
-// refinement's FP32 sweeps, the preconditioner made from the matrix as it is
-// now, and the matrix symmetric to the last bit (one flag, read back).
+// The symmetry stamp of the matrix (xcal_eqn::asym): read_asym enqueues its
+// read-back, asym_known takes it once the stream has been waited for.
 template <class T>
-static bool split_applies(Solver<T>& S, int precon) {
-  const xcal_eqn* e = S.e;
-  if (precon != XCAL_PRECON_DILU || !S.m->cone || !S.m->split || S.pc32 ||
+static void read_asym(Solver<T>& S) {
+  XCAL_HIP(hipMemcpyAsync(S.m->ctx->host_pinned + 60, S.e->asym.p, sizeof(int32_t),
+                          hipMemcpyDeviceToHost, S.s));
+}
+template <class T>
+static void asym_known(Solver<T>& S) {
+  int32_t stamp;
+  std::memcpy(&stamp, S.m->ctx->host_pinned + 60, sizeof stamp);
+  S.e->asym_host = stamp == (int32_t)S.e->precon_count;
+  S.e->asym_read = S.e->precon_count;
+}
+
+// Whether a CG solve starts in the split form: cone mesh with its tables, FP64
+// or refinement's FP32 sweeps, the preconditioner made from the matrix as it
+// is now, and the matrix symmetric to the last bit.  Where that is not known
+// yet the last one's answer is taken: a symmetric one's solve starts and reads
+// the stamp with its first state, another's reads it first.  A solve of at
+// most one iteration does not pay for the factors (1M cells, with the
+// preconditioner's update: one iteration 493 us classical, 580 split, two 719
+// and 698).
+template <class T>
+static bool split_applies(Solver<T>& S, int precon, int itmax) {
+  xcal_eqn* e = S.e;
+  if (precon != XCAL_PRECON_DILU || !S.m->cone || !S.m->split || S.pc32 || itmax < 2 ||
       e->precon_gen != e->nz_gen || e->asym.n < 1)
     return false;
-  int32_t* flag = (int32_t*)(S.m->ctx->host_pinned + 60);
-  XCAL_HIP(hipMemcpyAsync(flag, e->asym.p, sizeof(int32_t), hipMemcpyDeviceToHost, S.s));
-  XCAL_HIP(hipStreamSynchronize(S.s));
-  return *flag == 0;
+  if (e->asym_host && e->asym_read != e->precon_count) {
+    read_asym(S);
+    XCAL_HIP(hipStreamSynchronize(S.s));
+    asym_known(S);
+  }
+  return !e->asym_host;
 }
 
 // The split form's iterations (sweep_split.h), from the residual r and x = 0
 // (pa = 0): three launches each, the scalar updates done by the next kernel.
 // Its vectors are in the split row order: r and 1/D are brought to it here,
-// x (in it) is left for k_split_out.  Returns the final state.
+// x (in it) is left for k_split_out; `st` is the final state.  False, with r,
+// x and pa untouched, where the matrix turns out not to be symmetric.
 template <class T>
-static KS cg_split(Solver<T>& S, T* w) {
+static bool cg_split(Solver<T>& S, T* w, KS& st) {
   const int64_t n = S.n;
   const xcal_mesh* m = S.m;
   T *r = w, *x = w + n, *pa = w + 2 * n, *pb = w + 3 * n, *q = w + 4 * n, *t = w + 5 * n,
     *rho = w + 6 * n, *rD = w + 8 * n, *u0 = w + 9 * n;
-  const SplitFactors<T> f = split_factors(S.e, T(0));
+  xcal_eqn::Split<T>& f = split_of(S.e, T(0));
+  split_factors_f(S.e, f);
   const std::vector<int32_t>&bf = m->cone_f.band, &bb = m->cone_b.band;
   T* wv = bf.size() > 2 ? w + 7 * n : nullptr;  // later bands read w as their halo
   const int nf = m->cone_f.nblk(), vg = pfin_grid((int)grid_for(n));
@@ -1132,7 +1157,6 @@ static KS cg_split(Solver<T>& S, T* w) {
                        m->split_rows.p, v, out);
   };
   order(r, u0);
-  order(S.rD, rD);
   // the sweep's partials and the vector pass's, used in turn
   double *p0 = S.partial, *p1 = S.partial + 2 * (int64_t)nf;
   KS* cur = S.ks;
@@ -1142,8 +1166,8 @@ static KS cg_split(Solver<T>& S, T* w) {
       for (size_t k = 0; k + 1 < bf.size(); ++k)
         hipLaunchKernelGGL((k_split_fwd<decltype(start)::value, decltype(J)::value, T>),
                            dim3(bf[k + 1] - bf[k]), dim3(kConeBlock), 0, S.s,
-                           split_k(m->cone_f, bf[k]), f.a, f.f, u, (const T*)t, out, wv, n, p0,
-                           (const KS*)cur);
+                           split_k(m->cone_f, bf[k]), (const T*)f.a.p, (const T*)f.f.p, u,
+                           (const T*)t, out, wv, n, p0, (const KS*)cur);
     });
   };
   fwd(std::true_type{}, (const T*)u0, rho);
@@ -1161,8 +1185,9 @@ static KS cg_split(Solver<T>& S, T* w) {
       with_split_pairs(m->cone_b, [&](auto J) {
         for (size_t k = 0; k + 1 < bb.size(); ++k)
           hipLaunchKernelGGL((k_split_bwd<decltype(J)::value, T>), dim3(bb[k + 1] - bb[k]),
-                             dim3(kConeBlock), 0, S.s, split_k(m->cone_b, bb[k]), f.b, f.d,
-                             (const T*)rho, (const T*)pold, pnew, t, n, k == 0 ? Kb : Kn);
+                             dim3(kConeBlock), 0, S.s, split_k(m->cone_b, bb[k]),
+                             (const T*)f.b.p, (const T*)f.d.p, (const T*)rho, (const T*)pold,
+                             pnew, t, n, k == 0 ? Kb : Kn);
       });
     });
     cur = other(cur);
@@ -1173,8 +1198,16 @@ static KS cg_split(Solver<T>& S, T* w) {
                        (const T*)q, (const T*)rD, x, rho, p1, Kv);
     pend = true;
   };
-  KS st = read_state(S);
-  if (st.stop == STOP_NONE)
+  const bool known = S.e->asym_read == S.e->precon_count;
+  if (!known) read_asym(S);
+  st = read_state(S);
+  if (!known) {
+    asym_known(S);
+    if (S.e->asym_host) return false;
+  }
+  if (st.stop == STOP_NONE) {
+    split_factors_b(S.e, f, S.rD);
+    order(S.rD, rD);
     run_batches(S, S.cg_batch, 4, iteration, st, [&] {
       if (pend)  // an iteration leaves the state in S.ks, its last finalize pending
         hipLaunchKernelGGL(k_finalize_to, dim3(1), dim3(kBlock), 0, S.s, (const double*)p1, vg,
@@ -1182,8 +1215,9 @@ static KS cg_split(Solver<T>& S, T* w) {
       pend = false;
       cur = S.ks;
     });
+  }
   XCAL_HIP(hipGetLastError());
-  return st;
+  return true;
 }
 
 // Krylov.jl cg! with warm start x0 (solution = x0 + correction, written to
@@ -1199,8 +1233,9 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
   init_state(S, itmax, atol, rtol);
   hipLaunchKernelGGL(k_start<T>, dim3(S.gridA), dim3(kBlock), 0, S.s, S.A, b, (const T*)x0, r, x, pa);
   const bool dilu = precon == XCAL_PRECON_DILU;
-  if (split_applies(S, precon)) {
-    const KS st = cg_split(S, w);
+  KS st{};
+  const bool split_start = split_applies(S, precon, itmax);
+  if (split_start && cg_split(S, w, st)) {
     const int32_t* rows = S.m->split_rows.p;
     if (x0) hipLaunchKernelGGL((k_split_out<true, T>), dim3(S.grid), dim3(kBlock), 0, S.s, n, rows,
                                (const T*)x, x0);
@@ -1213,6 +1248,10 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
     niter = st.iter;
     return (st.stop == STOP_ITMAX || niter >= itmax) ? 1 : 0;
   }
+  if (split_start) {
+    st = KS{};
+    init_state(S, itmax, atol, rtol);
+  }
   const T* Sd = precon == XCAL_PRECON_JACOBI ? S.Sj : nullptr;
   const int sweep_slots = S.m->sweep_slots;
   if (dilu) {
@@ -1224,7 +1263,6 @@ static int cg(Solver<T>& S, int precon, const T* b, T* x0, int itmax, double ato
                        r, zd, (const T*)nullptr, S.partial);
     finalize_launch(S, S.grid, FIN_CG_INIT);
   }
-  KS st{};
   if (!dilu) {  // small meshes: the whole solve in one resident launch (persist.h)
     ResidentLease lease;
     if (persist_cg(S.e, S.A, Sd, x, (const T*)r, zd, S.ks, lease)) {

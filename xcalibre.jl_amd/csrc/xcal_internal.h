@@ -363,13 +363,23 @@ struct xcal_eqn {
   xcal::DBuf<double> Lrd;  // 1/D of each packed lower entry's column (0 on padding)
   xcal::DBuf<double> Lprod;  // a_ij a_ji of each packed lower entry (DILU diagonal update)
   // split CG on cone meshes: entry pairs of both sweeps, (1/D, a_ii - D) per
-  // forward and 1/D per backward position; asym != 0: A is not symmetric
-  xcal::DBuf<double> spa, spb, spf, spd;
-  xcal::DBuf<float> spa32, spb32, spf32, spd32;
+  // forward and 1/D per backward position, and the update they are of
+  template <class T>
+  struct Split {
+    xcal::DBuf<T> a, b, f, d;
+    int64_t gen_f = -1, gen_b = -1;
+  };
+  Split<double> split;
+  Split<float> split32;
+  // asym holds the last update (precon_count) whose matrix was not symmetric;
+  // asym_host: whether that of update asym_read was, as read back
   xcal::DBuf<int32_t> asym;
+  bool asym_host = false;
+  int64_t asym_read = -1;
   // changes of nzval, and their count at the last preconditioner update: the
   // split CG takes A's triangles from the preconditioner's factors
   int64_t nz_gen = 0, precon_gen = -1;
+  int64_t precon_count = 0;  // preconditioner updates on a cone mesh
   xcal::DBuf<double> La, Ua, Lp;  // lean sweeps: a_ij of both, a_ij a_ji of the lower entries
   xcal::DBuf<float> La32, Ua32;
   // cone form: a_ij and 1/D_j per forward cone entry, a_ij per backward cone
