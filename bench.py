@@ -562,7 +562,7 @@ def run_piso(args, x):
                    "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": hbm_traffic(args.roofline_kernel, f"channel_{N}cubed_fp64"),
+                     "traffic": hbm_traffic(args.roofline_kernel, f"channel_{N}cubed_fp64", split),
                      "kernel": args.roofline_kernel, "bytes_per_launch": nbytes,
                      "timed_launches": launches, "avg_us": round(avg_s * 1e6, 2)},
         "cpu_baseline": None,
@@ -594,12 +594,16 @@ def run_calib(args):
                       "launches": 3}))
 
 
-def hbm_traffic(kernel, workload):
+def hbm_traffic(kernel, workload, split=False):
     """HBM bytes per launch of `kernel` on `workload` from the committed
     rocprofv3 --pmc summary (L2-to-memory read requests by size, plus
     WRITE_SIZE, calibrated against a copy kernel), or None when no summary
-    covers this pair."""
+    covers this pair.  split: the sweeps are the split-preconditioned CG's,
+    other kernels than the classical iteration's, with summaries of their
+    own."""
     import re
+    if split:
+        kernel = kernel.replace("dilu_", "split_")
     path = ROOT / "profiles" / f"hbm_traffic_{kernel}_{workload}.md"
     if not path.exists():
         return None
@@ -758,7 +762,7 @@ def main():
         achieved = nbytes / avg_s / 1e9
         return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                "traffic": hbm_traffic(k, f"channel_{N}cubed_{args.precision}"),
+                "traffic": hbm_traffic(k, f"channel_{N}cubed_{args.precision}", split),
                 "kernel": k, "bytes_per_launch": nbytes, "timed_launches": launches,
                 "avg_us": round(avg_s * 1e6, 2)}
     # the dominant kernel: most time per CG iteration (every timed kernel
