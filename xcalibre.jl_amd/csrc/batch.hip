@@ -847,8 +847,8 @@ static std::vector<uint64_t> graph_key(const BSolver<T>& S, int kind, int precon
   const xcal_mesh* m = S.m;
   return {(uint64_t)kind, sizeof(T), (uint64_t)precon, (uint64_t)S.n, (uint64_t)S.ncase,
           (uint64_t)S.nblk, u(S.s), u(S.work), u(S.ks), u(S.partial), u(S.A.nz), u(S.A.colval),
-          u(S.A.rb), u(S.Sj), u(S.rD), u(S.Lnz), u(S.Unz), u(S.Db), u(S.Lrd), u(b),
-          (uint64_t)m->pipe_rw_f, (uint64_t)m->pipe_rw_b, (uint64_t)m->pipe_wf,
+          u(S.A.rb), u(S.Sj), u(S.rD), u(S.Lnz), u(S.Unz), u(S.Db), u(S.Lrd), u(S.La), u(S.Ua),
+          u(b), (uint64_t)m->pipe_rw_f, (uint64_t)m->pipe_rw_b, (uint64_t)m->pipe_wf,
           (uint64_t)m->pipe_wb};
 }
 
