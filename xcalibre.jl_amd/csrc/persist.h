@@ -32,12 +32,12 @@
 // case's result only where the state has stopped and is not marked
 // (resident_done); otherwise it solves by launches from the start.
 //
-// Measured per CG iteration on one MI355X, launch chain then resident (2D
-// k-omega steps, Jacobi): 8.8k rows 11.9 to 5.5 us, 130.7k rows 17.2 to 5.2
-// us, a batch of four (98k rows) 11.9 to 5.8 us.  What is left is the two
-// meetings, 1.0 us each for the flags alone and about 2 us with the sums, the
-// spread of the workgroups and the scalar update; the matrix is read once per
-// solve.
+// Measured per CG iteration on one MI355X (400 iterations of a solve, 2D
+// cavities, Jacobi, FP64), launch chain then resident: 8.8k rows 9.5 to 4.6 us,
+// 32k 9.6 to 5.6, 65k 9.9 to 6.1, 130k 15.4 to 7.2, 262k 19.7 to 9.1; a batch
+// of four (99k rows) 10.8 to 6.1.  What is left is the two meetings, 1.0 us
+// each for the flags alone and about 2 us with the sums, the spread of the
+// workgroups and the scalar update; the matrix is read once per solve.
 #pragma once
 
 #include "solver_common.h"

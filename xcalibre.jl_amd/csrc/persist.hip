@@ -7,13 +7,15 @@
 namespace xcal {
 
 // Rows a resident solve may have: at two rows per thread on every one of 256
-// compute units, and the 1024 slots of kPersistSlots for one case.  The gain
-// grows up to there (110.9k-row cavity 15.1 to 8.2 ms per 5 SIMPLE
-// iterations), so the line is what fits.
+// compute units, and the 1024 slots of kPersistSlots for one case.  It gains up
+// to there (262 144 rows 19.7 to 9.1 us per iteration), so the line is what
+// fits.
 constexpr int64_t kPersistRows = 1 << 18;
 // One row per thread up to this many workgroups, two above: fewer lines to
-// read per meeting (98 workgroups at two rows 24.1 ms, 195 at one 23.9 ms per
-// pass of the four-case batch; 130.7k rows 21.4 ms at 128 and 26 ms at 256).
+// read per meeting against more work between them.  Per iteration of a single
+// mesh, one row then two: 79 and 40 workgroups 5.83 and 5.99 us, 104 and 52
+// 6.15 and 6.07, 128 and 64 6.38 and 6.10, 188 and 94 7.45 and 6.68, 254 and
+// 127 7.80 and 7.22.
 constexpr int kPersistWide = 64;
 
 struct PersistPlan {

@@ -22,8 +22,8 @@
 // 256 threads.  Where every level has at most 256 rows the row-to-thread map
 // is the pipelined sweeps', so the dot products match theirs; where some have
 // more, k_plan_dots sums them in the launch form's order.  The rows' own sums
-// keep the reference's column order, so the sweep
-// equals the sequential loops (preconditioners_1_DILU.jl:43-114) bit for bit.
+// keep the reference's column order, so the sweep equals the sequential loops
+// (preconditioners_1_DILU.jl:43-114) bit for bit.
 //
 // Measured per forward / backward sweep on one MI355X, pipelined or launch
 // form then lean: 1600-cell cavity (79 levels) 25 / 25 to 15 / 17 us; 50k-cell
@@ -50,7 +50,7 @@ __device__ inline void opaque(V& v) {
 
 // One sweep direction (device arrays of xcal_mesh::Lean).  W entries per row.
 struct LeanK {
-  const int2* steps;      // first position, rows (0: a padding step); groups of kLeanGroup
+  const int2* steps;      // first position, rows (0: a padding step); groups of kLeanDepth
   const int32_t* cstep;   // first step of each case (ncase + 1)
   const uint32_t* idx;    // W = 2: one word of two slots per position; W = 3: two words
   int64_t n;              // positions (third entries follow the 2 n pairs)
