@@ -71,7 +71,12 @@ def test_split_cg_equals_classical_cg(x, A, ctx, monkeypatch, name, prec):
     b = _solve(x, A, ctx, mesh, monkeypatch, True, prec)
     for u, v in zip(a, b):
         assert u[1] == v[1] == 0
-        assert abs(u[0] - v[0]) <= (2 if prec == "PREC_FP64" else 6), (u[0], v[0])
+        # Refinement's FP32 solves: the two forms' matrices differ by FP32's
+        # rounding, so what a sweep loses to it differs, by less than half a
+        # decimal digit of the residual; a digit takes a tenth of a solve to
+        # 1e-10 (measured 585 against 596 iterations at most, the split form
+        # holding A's diagonal more exactly than FP32 does).
+        assert abs(u[0] - v[0]) <= (2 if prec == "PREC_FP64" else max(6, v[0] // 20)), (u[0], v[0])
     assert rel(a[1][2], b[1][2]) < 1e-9
     assert not np.array_equal(a[0][2], b[0][2])  # the split form ran
 
@@ -137,3 +142,43 @@ def test_split_cg_follows_the_matrix_from_update_to_update(x, A, ctx, monkeypatc
         else:  # twelve iterations' rounding, in the sweeps' precision
             assert rel(u[4], v[4]) < (1e-12 if prec == "PREC_FP64" else 1e-4)
             assert not np.array_equal(u[4], v[4])
+
+
+def test_split_refinement_solves_the_matrix_as_it_is(x, A, ctx, monkeypatch):
+    """FP32 solves of refinement where rounding the factors matters: a uniform
+    cavity whose coefficients jump between 1 and 1/100.  A's diagonal, which the
+    split sweeps make of two FP32 values, has to stay A's to far below FP32's
+    rounding, or refinement converges towards it slowly: with the two rounded
+    apart the solves took 2.1 times the classical form's inner iterations in
+    all, chosen together 1.08 times (0.94 to 1.24 for single systems)."""
+    H = x.hip
+    mesh = _mesh(x, "quad")
+    fc = np.asarray(mesh.face_centre).reshape(mesh.n_faces, 3)
+    total = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("XCAL_NO_SPLIT", "1")
+        dm = H.DeviceMesh(ctx, mesh)
+        monkeypatch.delenv("XCAL_NO_SPLIT", raising=False)
+        its = 0
+        for seed in range(3):
+            rng = np.random.default_rng(100 + seed)
+            a, b = rng.uniform(3, 12, 2)
+            high = np.sin(a * fc[:, 0] + seed) * np.cos(b * fc[:, 1]) > 0
+            g = H.Field(dm, A.FACE_SCALAR).upload(np.where(high, 1.0, 0.01))
+            s = H.Field(dm, A.CELL_SCALAR).upload(rng.standard_normal(mesh.n_cells))
+            phi = H.Field(dm, A.CELL_SCALAR)
+            eq = H.Equation(dm, False)
+            terms = [(A.LAPLACIAN_LINEAR, -1, g)]
+            bcs = A.bc_array([(A.BC_DIRICHLET if i == 0 else A.BC_ZEROGRADIENT, i, 0.0)
+                              for i in range(len(mesh.patch_names))])
+            eq.discretise(terms, [(s, 1)])
+            eq.apply_bcs(terms, bcs, phi)
+            eq.precond_update(A.PRECON_DILU)
+            n, _, rc = eq.solve(A.SolverSetupC(A.SOLVER_CG, A.PRECON_DILU, A.PREC_FP32_IR, 4000,
+                                               1e-7, 1.0, 0.0, 1e-10, 1e-6, 0, 0.0), phi)
+            assert rc == 0
+            its += n
+        total.append(its)
+    print(f"inner iterations: split {total[0]}, classical {total[1]}")
+    assert total[0] <= 1.3 * total[1]

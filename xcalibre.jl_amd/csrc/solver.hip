@@ -449,18 +449,53 @@ __global__ void __launch_bounds__(kBlock)
   const int32_t i = rows[p];
   out[i] = ADD ? out[i] + x[p] : x[p];
 }
-// (1/D, a_ii - D) per forward cone position
+// The diagonal of the split form per row: 1/D and a_ii - D.  The sweeps make
+// A's diagonal of the two, as the reciprocal of the first plus the second, so
+// in FP32 they are chosen together: of the 33 values around 1/D (a change of
+// D that small is nothing to the preconditioner) the one whose remainder
+// a_ii - 1/(1/D) is nearest to an FP32 value, which leaves some 1e-10 of a_ii.
+// Rounded apart they leave up to 1e-7, of one sign where the coefficients are
+// uniform, and the refinement's FP32 solves are of another matrix: on a 300x300
+// uniform cavity with coefficients of 1 and 1/1000 they took 2940 to more than
+// 4000 inner iterations so, 1490 to 1727 now, and 1477 to 1757 classically.
 template <class T>
 __global__ void __launch_bounds__(kBlock)
-    k_split_scalars(int64_t total, const int32_t* __restrict__ crow,
-                    const int32_t* __restrict__ diag, const double* __restrict__ nz,
-                    const double* __restrict__ D, const double* __restrict__ rD,
-                    T* __restrict__ out) {
+    k_split_diag(int64_t n, const int32_t* __restrict__ diag, const double* __restrict__ nz,
+                 const double* __restrict__ D, T* __restrict__ rd, T* __restrict__ rest) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double a = nz[diag[i]], d = D[i];
+  const T r0 = (T)(1.0 / d);
+  if constexpr (sizeof(T) == 8) {
+    rd[i] = r0;
+    rest[i] = a - d;
+  } else {
+    T r = r0, s = (T)(a - 1.0 / (double)r0);
+    double err = fabs(a - 1.0 / (double)r - (double)s);
+    for (int k = -16; k <= 16; ++k) {
+      const T rk = __int_as_float(__float_as_int(r0) + k);
+      const double e = a - 1.0 / (double)rk;
+      const T sk = (T)e;
+      if (fabs(e - (double)sk) < err) {
+        err = fabs(e - (double)sk);
+        r = rk;
+        s = sk;
+      }
+    }
+    rd[i] = r;
+    rest[i] = s;
+  }
+}
+// the two per forward cone position
+template <class T>
+__global__ void __launch_bounds__(kBlock)
+    k_split_scalars(int64_t total, const int32_t* __restrict__ crow, const T* __restrict__ rd,
+                    const T* __restrict__ rest, T* __restrict__ out) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= total) return;
   const int32_t c = crow[p], i = c >= 0 ? c : ~c;
-  out[2 * p] = (T)rD[i];
-  out[2 * p + 1] = (T)(nz[diag[i]] - D[i]);
+  out[2 * p] = rd[i];
+  out[2 * p + 1] = rest[i];
 }
 
 // b = 1 / a rounded to FP32
@@ -1035,22 +1070,27 @@ static void split_factors_f(xcal_eqn* e, xcal_eqn::Split<T>& f) {
   const xcal_mesh::Cone& F = m->cone_f;
   split_pairs(e, f.a, F.pslot);
   if (f.f.n != 2 * F.rows) f.f.alloc(2 * F.rows);
+  if (f.rd.n != m->n) {
+    f.rd.alloc(m->n);
+    f.rest.alloc(m->n);
+  }
+  hipLaunchKernelGGL(k_split_diag<T>, dim3(grid_for(m->n)), dim3(kBlock), 0, m->ctx->stream, m->n,
+                     m->diag.p, (const double*)e->nzval.p, (const double*)e->pD.p, f.rd.p,
+                     f.rest.p);
   hipLaunchKernelGGL(k_split_scalars<T>, dim3(grid_for(F.rows)), dim3(kBlock), 0, m->ctx->stream,
-                     F.rows, F.crow.p, m->diag.p, (const double*)e->nzval.p,
-                     (const double*)e->pD.p, (const double*)e->prD.p, f.f.p);
+                     F.rows, F.crow.p, (const T*)f.rd.p, (const T*)f.rest.p, f.f.p);
   XCAL_HIP(hipGetLastError());
   f.gen_f = e->precon_count;
 }
-// rD: the preconditioner's 1/D in T
 template <class T>
-static void split_factors_b(xcal_eqn* e, xcal_eqn::Split<T>& f, const T* rD) {
+static void split_factors_b(xcal_eqn* e, xcal_eqn::Split<T>& f) {
   if (f.gen_b == e->precon_count) return;
   const xcal_mesh* m = e->mesh;
   const xcal_mesh::Cone& B = m->cone_b;
   split_pairs(e, f.b, B.pslot);
   if (f.d.n != B.rows) f.d.alloc(B.rows);
   hipLaunchKernelGGL(k_split_rows<T>, dim3(grid_for(B.rows)), dim3(kBlock), 0, m->ctx->stream,
-                     B.rows, B.crow.p, rD, f.d.p);
+                     B.rows, B.crow.p, (const T*)f.rd.p, f.d.p);
   XCAL_HIP(hipGetLastError());
   f.gen_b = e->precon_count;
 }
@@ -1206,8 +1246,8 @@ static bool cg_split(Solver<T>& S, T* w, KS& st) {
     if (S.e->asym_host) return false;
   }
   if (st.stop == STOP_NONE) {
-    split_factors_b(S.e, f, S.rD);
-    order(S.rD, rD);
+    split_factors_b(S.e, f);
+    order((const T*)f.rd.p, rD);
     run_batches(S, S.cg_batch, 4, iteration, st, [&] {
       if (pend)  // an iteration leaves the state in S.ks, its last finalize pending
         hipLaunchKernelGGL(k_finalize_to, dim3(1), dim3(kBlock), 0, S.s, (const double*)p1, vg,

@@ -363,10 +363,11 @@ struct xcal_eqn {
   xcal::DBuf<double> Lrd;  // 1/D of each packed lower entry's column (0 on padding)
   xcal::DBuf<double> Lprod;  // a_ij a_ji of each packed lower entry (DILU diagonal update)
   // split CG on cone meshes: entry pairs of both sweeps, (1/D, a_ii - D) per
-  // forward and 1/D per backward position, and the update they are of
+  // forward and 1/D per backward position, the same two per row, and the
+  // update they are of
   template <class T>
   struct Split {
-    xcal::DBuf<T> a, b, f, d;
+    xcal::DBuf<T> a, b, f, d, rd, rest;
     int64_t gen_f = -1, gen_b = -1;
   };
   Split<double> split;
